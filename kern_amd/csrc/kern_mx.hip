@@ -615,166 +615,6 @@ GEMV_PERSISTENT(7)
 GEMV_PERSISTENT(8)
 #undef GEMV_PERSISTENT
 
-// ------------------------------------- dense MXFP4 x MXFP8 -> bf16 at M <= 64 tokens: the persistent walk
-// The tiled GEMM gives a small batch one workgroup per 256 weight rows (36 at N = 9216, which read the
-// weights at about 1.2 TB/s). This kernel walks the weights as gemv_persistent does (about 256 workgroups
-// of 8 waves, hb <= 9 half groups each, wave w owning k-tiles [w*KTW, (w+1)*KTW) of K = 1024*KTW, k-tile
-// by k-tile across the row groups, fragments four ahead) and multiplies them in their fp4 form on the
-// block-scaled MFMA against the MXFP8 activations of four 16-token groups. Lane (c, q) of group tg takes
-// token 16*tg + c's bytes [16q, 16q + 16) and [64 + 16q, +16) of the k-tile (the 8-bit operand layout of
-// V_MFMA_SCALE_F32_16X16X128_F8F6F4) and its k block q's scale byte, both through the wave's LDS: the
-// k-tile's rows are requested row-contiguous one k-tile ahead, and the scale bytes of the wave's k groups
-// once. Requested straight in operand pieces, each request gathered 16 rows (M = 64, N = 9216: 25.8
-// against 17.0 us). Both scale operands arrive shifted to byte 0 (OPSEL 0). The eight partial sums meet
-// in LDS one token group at a time; dbg (if not null) receives the f32 sums the bf16 values round.
-template <int KTW>
-KERN_DEV void gemm_skinny_bf16(const uint8_t* __restrict__ w, const uint8_t* __restrict__ wsf,
-                               const uint8_t* __restrict__ xq, const uint8_t* __restrict__ xsf,
-                               uint16_t* __restrict__ y, float* __restrict__ dbg, int M, int N, int K, int hb) {
-  constexpr int NG = 5, D = 4, TOT = NG * KTW, TG = 4;
-  constexpr int NS = (KTW + 6) / 4;  // k groups a wave's k-tiles touch (KTW <= 8: at most three)
-  __shared__ v4f red[8][NG][64];
-  __shared__ __attribute__((aligned(16))) uint8_t xst[8][8192];      // per wave: one k-tile of 64 token rows
-  __shared__ __attribute__((aligned(16))) uint8_t sst[8][NS][1024];  // per wave: 64 rows' 16 scale bytes a k group
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int KT = K >> 7, KG = K >> 9, KB = K >> 5;
-  const int H = N >> 3;
-  const int h0 = blockIdx.x * hb, h1 = min(h0 + hb, H);
-  const int g0 = h0 >> 1, ng = ((h1 + 1) >> 1) - g0;  // row groups touched: [g0, g0 + ng), ng <= NG
-  const int c = lane & 15, q = lane >> 4, r = lane & 15;
-  const int kt0 = wave * KTW, kgA = kt0 >> 2;
-  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)xq, (short)0, M * K, 0x00020000);
-  const __amdgpu_buffer_rsrc_t xsr = __builtin_amdgcn_make_buffer_rsrc((void*)xsf, (short)0, M * KB, 0x00020000);
-  // activations are requested row-contiguous: request p of a k-tile loads token rows 8p .. 8p+7, 8 lanes a
-  // 128-byte row; they pass through the wave's LDS (16-byte chunk h of row r at h ^ ((r >> 1) & 7)) and are
-  // read back as operand pieces. Scale bytes: the wave's NS k groups, one 16-byte request per row each,
-  // staged once. Absent tokens and k groups read zeros; requests with no present token are not sent (their
-  // LDS rows reach only the MFMA columns of absent tokens, never stored).
-  int xo[8];
-#pragma unroll
-  for (int p = 0; p < 8; ++p) {
-    const int row = 8 * p + (lane >> 3);
-    xo[p] = row < M ? row * K + 128 * kt0 + 16 * (lane & 7) : 0x40000000;
-  }
-  v4u xl[8];
-  auto load_x = [&](int j) {
-#pragma unroll
-    for (int p = 0; p < 8; ++p)
-      if (8 * p < M) xl[p] = __builtin_amdgcn_raw_buffer_load_b128(xr, xo[p] + 128 * j, 0, 0);
-  };
-  {
-    v4u sl[NS];
-#pragma unroll
-    for (int t = 0; t < NS; ++t)
-      sl[t] = __builtin_amdgcn_raw_buffer_load_b128(xsr, (lane < M && kgA + t < KG) ? lane * KB + 16 * (kgA + t)
-                                                                                      : 0x40000000, 0, 0);
-#pragma unroll
-    for (int t = 0; t < NS; ++t) *reinterpret_cast<v4u*>(&sst[wave][t][lane * 16]) = sl[t];
-    WAVE_LDS_SYNC();
-  }
-  load_x(0);
-  v4u xa[TG], xb[TG];
-  // weight-scale dwords of k groups kgA .. kgA + 2 (KTW <= 8 consecutive k-tiles span at most three groups)
-  const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(wsf + (int64_t)g0 * KG * 256), (short)0, ng * KG * 256, 0x00020000);
-  uint32_t sdw[NG][NS];
-#pragma unroll
-  for (int g = 0; g < NG; ++g)
-#pragma unroll
-    for (int t = 0; t < NS; ++t) {
-      const int kg = kgA + t;
-      sdw[g][t] = __builtin_amdgcn_raw_buffer_load_b32(
-          sr, (g < ng && kg < KG) ? (g * KG + kg) * 256 + lane * 4 : 0x40000000, 0, 2);
-    }
-  const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(w + (int64_t)g0 * KT * 1024), (short)0, ng * KT * 1024, 0x00020000);
-  // item i = j*NG + g is fragment (g0 + g, kt0 + j); rows outside the owned half groups read zeros
-  auto woff = [&](int i) -> int {
-    const int g = i % NG, half = (g0 + g) * 2 + (r >> 3);
-    return (g < ng && half >= h0 && half < h1) ? (g * KT + kt0 + i / NG) * 1024 + lane * 16 : 0x40000000;
-  };
-  v4u buf[D];
-#pragma unroll
-  for (int i = 0; i < D; ++i) {
-    if (i < TOT) buf[i] = __builtin_amdgcn_raw_buffer_load_b128(wr, woff(i), 0, 2);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  v4f acc[NG][TG] = {};
-#pragma unroll
-  for (int i = 0; i < TOT; ++i) {
-    const int g = i % NG, j = i / NG, kt = kt0 + j;
-    uint32_t xs[TG];
-    if (g == 0) {
-#pragma unroll
-      for (int p = 0; p < 8; ++p) {
-        const int row = 8 * p + (lane >> 3);
-        if (8 * p < M) *reinterpret_cast<v4u*>(&xst[wave][row * 128 + (((lane & 7) ^ ((row >> 1) & 7)) << 4)]) = xl[p];
-      }
-      WAVE_LDS_SYNC();
-#pragma unroll
-      for (int tg = 0; tg < TG; ++tg) {
-        const int row = 16 * tg + c, sw = (row >> 1) & 7;
-        xa[tg] = *reinterpret_cast<const v4u*>(&xst[wave][row * 128 + ((q ^ sw) << 4)]);
-        xb[tg] = *reinterpret_cast<const v4u*>(&xst[wave][row * 128 + (((q + 4) ^ sw) << 4)]);
-      }
-      if (j + 1 < KTW) load_x(j + 1);
-    }
-#pragma unroll
-    for (int tg = 0; tg < TG; ++tg)
-      xs[tg] = *reinterpret_cast<const uint32_t*>(&sst[wave][(kt >> 2) - kgA][(16 * tg + c) * 16 + 4 * (kt & 3)]);
-    const v4u wv = buf[i % D];
-    if (g == 0 || g < ng) {
-      const int sw = (int)(sdw[g][(kt >> 2) - kgA] >> (8 * (kt & 3)));
-      const v8i a = {(int)wv[0], (int)wv[1], (int)wv[2], (int)wv[3], 0, 0, 0, 0};
-#pragma unroll
-      for (int tg = 0; tg < TG; ++tg) {
-        if (16 * tg >= M) break;  // token groups with no token (uniform)
-        const v4u lo = xa[tg], hi = xb[tg];
-        const v8i b = {(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
-        const int sx = (int)(xs[tg] >> (8 * q));
-        acc[g][tg] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, acc[g][tg], 4, 0, 0, sw, 0, sx);
-      }
-    }
-    if (i + D < TOT) buf[i % D] = __builtin_amdgcn_raw_buffer_load_b128(wr, woff(i + D), 0, 2);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-#pragma unroll
-  for (int tg = 0; tg < TG; ++tg) {
-    if (16 * tg >= M) break;
-#pragma unroll
-    for (int g = 0; g < NG; ++g) red[wave][g][lane] = acc[g][tg];
-    __syncthreads();
-    for (int g = wave; g < ng; g += 8) {
-      v4f s = red[0][g][lane];
-#pragma unroll
-      for (int v = 1; v < 8; ++v) s += red[v][g][lane];
-      const int half = (g0 + g) * 2 + (q >> 1), t = 16 * tg + c;
-      if (t < M && half >= h0 && half < h1) {
-        const int64_t o = (int64_t)t * N + (g0 + g) * 16 + q * 4;
-        const uint32_t lo = f32_to_bf16_bits(s[0]) | (f32_to_bf16_bits(s[1]) << 16);
-        const uint32_t hi = f32_to_bf16_bits(s[2]) | (f32_to_bf16_bits(s[3]) << 16);
-        *reinterpret_cast<uint2*>(y + o) = make_uint2(lo, hi);
-        if (dbg) *reinterpret_cast<v4f*>(dbg + o) = s;
-      }
-    }
-    __syncthreads();
-  }
-}
-
-#define GEMM_SKINNY(KTW)                                                                                       \
-  extern "C" __global__ __launch_bounds__(512) void kern_mx_gemm_bf16_s##KTW(                                   \
-      const uint8_t* __restrict__ w, const uint8_t* __restrict__ wsf, const uint8_t* __restrict__ xq,          \
-      const uint8_t* __restrict__ xsf, uint16_t* __restrict__ y, float* __restrict__ dbg, int M, int N, int K, \
-      int hb) {                                                                                                \
-    gemm_skinny_bf16<KTW>(w, wsf, xq, xsf, y, dbg, M, N, K, hb);                                               \
-  }
-GEMM_SKINNY(1)
-GEMM_SKINNY(2)
-GEMM_SKINNY(4)
-GEMM_SKINNY(7)
-GEMM_SKINNY(8)
-#undef GEMM_SKINNY
-
 // ====================================================================================== block-scaled GEMM
 // One workgroup computes a 128-row (token/slot) x 256-row (weight) tile with 8 waves (two per SIMD) in a
 // 2x4 grid; each wave owns 64 x 64 = 4 x 4 tiles of V_MFMA_SCALE_F32_16X16X128_F8F6F4 (A = fp4 weights,
@@ -1833,6 +1673,250 @@ extern "C" __global__ __launch_bounds__(512) void kern_mx_gemm_bf16(const uint8_
   A.m = m; A.k = k; A.rows = M; A.sf_b_r128c4 = 0; A.dbg = dbg;
   bmm_tile<MODE_DENSE_BF16>(A, L);
 }
+
+// ------------------------------------------- dense MXFP4 x MXFP8 of small and middle batches: small tiles
+// The ring's 128 x 256 tiles give a batch of M <= 128 rows one workgroup per 256 weight rows (16 at N = 4096),
+// so most of the chip idles until M * N holds some 200 of them. gemm_tiles covers the range below that: tiles of
+// 16*MT token rows x 16*NW*NF weight rows, one workgroup of NW waves each, wave w multiplying weight groups
+// [w*NF, +NF) of the tile with all of its token rows, k-tile after k-tile in one accumulator, so that every
+// result has the ring's bits. What bounds a tile is the operand bytes its CU can pull in (about 39 B a clock of the
+// 64 B the address path takes), so each operand byte is requested once per tile and many requests are in flight:
+//   * weight fragments go straight into registers (a wave is the only one to use its fragments) and with them a
+//     scale dword per fragment and k group, S k groups (of 512) ahead. Default cache policy: with three weight
+//     copies in turn (M = 200, N = 4096, K = 7168) non-temporal loads took 14.2 us against 11.5 (the token
+//     blocks of a weight tile share one L2, and the weights may still sit in the Infinity Cache); with 600 MB of
+//     copies in turn the two are within 5% (M = 64, N = 9216: 13.7 non-temporal, 14.4 default);
+//   * activations go through an LDS ring of S k groups by buffer->LDS requests (rows of 128 bytes, the ring
+//     GEMM's 16-byte chunk swizzle applied on the global side), S - 1 k groups ahead, each wave an equal share,
+//     with one barrier a k group;
+//   * the tile's token scales, one contiguous block of memory, are copied to LDS once at the start. Fetched
+//     per k group (16 bytes of each row) they took as long as the activations: 17.8 against 14.9 us.
+// The k groups take the last steps of whole rounds of S, so that the last round needs no requests and none runs
+// past the end; the first steps of the first round (at most S - 1) send theirs to a zero-length resource.
+// Measured against the ring (one process, graph replays, three weight copies in turn, us): M = 40, N = 6144,
+// K = 3584 12.5 -> 6.4; M = 200, N = 4096, K = 7168 29.6 -> 12.3; M = 200, N = 7168, K = 2048 12.5 -> 7.9;
+// M = 128, N = 9216, K = 7168 30.4 -> 15.4; M = 1024, N = 4096, K = 7168 33.4 -> 28.6. A form that split K over
+// four waves and added the partial sums in LDS was within 10% either way and rounds differently.
+template <int MT, int NW, int NF>
+struct TileCfg {
+  static constexpr int S = NW * NF <= 4 && MT <= 2 ? 8 : (MT >= 5 || NF >= 2 ? 3 : 4);  // stages: k groups in flight
+  static constexpr int NX = 8 * MT / NW;      // activation requests of a wave and k group
+  static constexpr int STAGE = MT * 8192;     // activations of one k group
+  static_assert((S - 1) * 5 * NF + (S - 2) * NX <= 63, "the stage's wait is a vmcnt");
+};
+
+template <int MODE, int MT, int NW, int NF>
+KERN_DEV void gemm_tiles(const uint8_t* __restrict__ w, const uint8_t* __restrict__ wsf, const uint8_t* __restrict__ xq,
+                       const uint8_t* __restrict__ xsf, void* __restrict__ y, const float* d_scale,
+                       float* __restrict__ dbg, int M, int N, int K) {
+  using C = TileCfg<MT, NW, NF>;
+  constexpr int S = C::S, TM = 16 * MT, NX = C::NX, NWL = 5 * NF;
+  extern __shared__ __attribute__((aligned(1024))) uint8_t tile_lds[];  // S stages, then the token scales
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, q = lane >> 4;
+  const int KT = K >> 7, KG = K >> 9, KB = K >> 5;
+  // tile: each XCD (workgroup lin on XCD lin % 8) takes a contiguous run of tiles, token blocks fastest, so
+  // that a weight tile's token blocks share one L2
+  const int total = gridDim.x * gridDim.y, lin = blockIdx.x + gridDim.x * blockIdx.y, xcd = lin & 7;
+  const int tile = xcd * (total >> 3) + min(xcd, total & 7) + (lin >> 3);
+  const int nt = tile / (int)gridDim.y, mt = tile - nt * (int)gridDim.y;
+  const int m0 = mt * TM, rows = min(TM, M - m0);
+  const int g0 = nt * NW * NF, ng = min(NW * NF, (N >> 4) - g0);  // the tile's 16-row weight groups
+  // the k groups take the last KG of a whole number of rounds of S steps: step v is k group v - p0
+  const int p0 = (S - KG % S) % S, V = KG + p0;
+  // the tile's token scales, [row][KB + 16] (the pad spreads the rows' reads over the banks)
+  uint8_t* xsc = tile_lds + S * C::STAGE;
+  {
+    const __amdgpu_buffer_rsrc_t sr =
+        __builtin_amdgcn_make_buffer_rsrc((void*)(xsf + (int64_t)m0 * KB), (short)0, rows * KB, 0x00020000);
+    const int P = (KB >> 4) + 1, pieces = TM * P;
+    for (int i0 = wave * 64; i0 < pieces; i0 += 64 * NW) {
+      const int i = i0 + lane, row = i / P, k = i - row * P;
+      const int off = row < rows && k < P - 1 ? row * KB + 16 * k : 0x7fffff00;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(sr, (lds_void_t*)(xsc + i0 * 16), 16, off, 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // buffer resources, of length zero for the steps before the first k group (zeros, no memory traffic)
+  const uint8_t* xb0 = xq + (int64_t)m0 * K;
+  const uint8_t* wb0 = w + (int64_t)g0 * KT * 1024;
+  const uint8_t* sb0 = wsf + (int64_t)g0 * KG * 256;
+  auto rsrc = [&](const void* base, int bytes, bool live) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, live ? bytes : 0, 0x00020000);
+  };
+  // request i of a wave: r = wave * NX + i of the k group's 8 * MT, k-tile r / (2 * MT), rows 8 * (r % (2 * MT))
+  // .. +8, 16 bytes a lane; rows past the batch lie past the resource's end (zeros)
+  int xo[NX];
+#pragma unroll
+  for (int i = 0; i < NX; ++i) {
+    const int row = 8 * ((wave * NX + i) % (2 * MT)) + (lane >> 3);
+    xo[i] = row < rows ? row * K + (((lane & 7) ^ ((row >> 1) & 7)) << 4) : 0x7fffff00;
+  }
+  int wo[NF], so[NF];
+#pragma unroll
+  for (int f = 0; f < NF; ++f) {
+    const int g = wave * NF + f;
+    wo[f] = g < ng ? g * KT * 1024 + lane * 16 : 0x7fff0000;
+    so[f] = g < ng ? g * KG * 256 + lane * 4 : 0x7fffff00;
+  }
+  auto dma = [&](int v, int slot) {
+    const __amdgpu_buffer_rsrc_t x_ = rsrc(xb0, rows * K, v >= p0);
+    const int kg = v - p0;
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      const int r = wave * NX + i;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(x_, (lds_void_t*)(tile_lds + slot * C::STAGE + r * 1024), 16, xo[i],
+                                               __builtin_amdgcn_readfirstlane((4 * kg + r / (2 * MT)) * 128), 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  v4u wv[S][NF][4];
+  uint32_t ws[S][NF];
+  auto load_w = [&](int v, auto Ic) {
+    constexpr int i = decltype(Ic)::value;
+    const __amdgpu_buffer_rsrc_t w_ = rsrc(wb0, ng * KT * 1024, v >= p0), s_ = rsrc(sb0, ng * KG * 256, v >= p0);
+    const int kg = v - p0;
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      ws[i][f] = __builtin_amdgcn_raw_buffer_load_b32(s_, so[f], __builtin_amdgcn_readfirstlane(kg * 256), 0);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        wv[i][f][j] = __builtin_amdgcn_raw_buffer_load_b128(w_, wo[f] + 1024 * j,
+                                                            __builtin_amdgcn_readfirstlane(kg * 4096), 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+  v4f acc[MT][NF];
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int f = 0; f < NF; ++f) acc[t][f] = (v4f){0.f, 0.f, 0.f, 0.f};
+  // requests in the order of the steady state: W(0), X(0), W(1), X(1), .. X(S - 2), W(S - 1)
+  auto prologue = [&](auto&& self, auto Ic) -> void {
+    constexpr int i = decltype(Ic)::value;
+    if constexpr (i < S) {
+      load_w(i, Ic);
+      if constexpr (i + 1 < S) dma(i, i);
+      self(self, IC<i + 1>{});
+    }
+  };
+  prologue(prologue, IC<0>{});
+  auto multiply = [&](int kg, auto Ic) {
+    constexpr int i = decltype(Ic)::value;
+    const uint8_t* st = tile_lds + i * C::STAGE;
+    v4u sx[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) sx[t] = *reinterpret_cast<const v4u*>(xsc + (16 * t + c) * (KB + 16) + 16 * kg);
+    auto ktile = [&](auto Jc) {
+      constexpr int j = decltype(Jc)::value;
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        const int row = 16 * t + c, z = (row >> 1) & 7;
+        const uint8_t* xrow = st + j * (TM * 128) + row * 128;
+        const v4i lo = *reinterpret_cast<const v4i*>(xrow + ((q ^ z) << 4));
+        const v4i hi = *reinterpret_cast<const v4i*>(xrow + (((q + 4) ^ z) << 4));
+        const v8i xb = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        const int sxb = (int)(sx[t][j] >> (8 * q));
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+          const v8i a = {(int)wv[i][f][j][0], (int)wv[i][f][j][1], (int)wv[i][f][j][2], (int)wv[i][f][j][3], 0, 0, 0, 0};
+          acc[t][f] =
+              __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, xb, acc[t][f], 4, 0, j, (int)ws[i][f], 0, sxb);
+        }
+      }
+    };
+    ktile(IC<0>{}), ktile(IC<1>{}), ktile(IC<2>{}), ktile(IC<3>{});
+  };
+  // step v (stage i): this wave's requests of step v's X have landed once only those sent after them are in
+  // flight; after the barrier every wave's have, and every wave has read step v - 1 (its multiplies consumed
+  // the reads), whose slot takes step v + S - 1. Before the last round W(v + 1 .. v + S - 1) and
+  // X(v + 1 .. v + S - 2) follow X(v); in it only the remaining steps' do.
+  auto step = [&](int v, auto Ic, auto LASTc) {
+    constexpr int i = decltype(Ic)::value;
+    constexpr bool LAST = decltype(LASTc)::value;
+    if constexpr (LAST && i > 0)
+      WAIT_VMCNT((S - 1 - i) * (NWL + NX));
+    else
+      WAIT_VMCNT((S - 1) * NWL + (S - 2) * NX);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (!LAST || i == 0) dma(v + S - 1, (i + S - 1) % S);
+    if (v >= p0) multiply(v - p0, Ic);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (!LAST) load_w(v + S, Ic);
+  };
+  auto round_ = [&](auto&& self, int v, auto Ic, auto LASTc) -> void {
+    constexpr int i = decltype(Ic)::value;
+    if constexpr (i < S) {
+      step(v + i, Ic, LASTc);
+      self(self, v, IC<i + 1>{}, LASTc);
+    }
+  };
+  int v = 0;
+  for (; v < V - S; v += S) round_(round_, v, IC<0>{}, IC<0>{});
+  round_(round_, v, IC<0>{}, IC<1>{});
+  float ds = 0.f;
+  if (MODE == MODE_PT) ds = d_scale[0];
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      const int g = wave * NF + f, row = 16 * t + c;
+      if (row < rows && g < ng) {
+        const v4f s = acc[t][f];
+        const int64_t o = (int64_t)(m0 + row) * N + (g0 + g) * 16 + 4 * q;
+        if (MODE == MODE_PT)
+          *reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(y) + o) =
+              e4m3_hw2(s[0] * ds, s[1] * ds) | (e4m3_hw2(s[2] * ds, s[3] * ds) << 16);
+        else
+          *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(y) + o) =
+              make_uint2(bf16x2_hw(s[0], s[1]), bf16x2_hw(s[2], s[3]));
+        if (dbg) *reinterpret_cast<v4f*>(dbg + o) = s;
+      }
+    }
+}
+
+// Entries: tile 16*MT x 16*NW*NF as t{rows}x{weights}, grid [ceil(N / weights), ceil(M / rows)], block 64 * NW,
+// dynamic LDS S * MT * 8 KiB + the token scales (16*MT rows of K/32 + 16 bytes, in whole KiB).
+#define GEMM_TILES(TM, TN, MT, NW, NF)                                                                         \
+  extern "C" __global__ __launch_bounds__(64 * NW) void kern_mx_gemm_bf16_t##TM##x##TN(                         \
+      const uint8_t* w, const uint8_t* wsf, const uint8_t* xq, const uint8_t* xsf, uint16_t* y, int M, int N,  \
+      int K, float* dbg) {                                                                                     \
+    gemm_tiles<MODE_DENSE_BF16, MT, NW, NF>(w, wsf, xq, xsf, y, nullptr, dbg, M, N, K);                        \
+  }                                                                                                            \
+  extern "C" __global__ __launch_bounds__(64 * NW) void kern_mx_gemm_e4m3_t##TM##x##TN(                         \
+      const uint8_t* w, const uint8_t* wsf, const uint8_t* xq, const uint8_t* xsf, uint8_t* y,                 \
+      const float* d_scale, int M, int N, int K, float* dbg) {                                                 \
+    gemm_tiles<MODE_PT, MT, NW, NF>(w, wsf, xq, xsf, y, d_scale, dbg, M, N, K);                                \
+  }
+GEMM_TILES(16, 32, 1, 2, 1)
+GEMM_TILES(16, 64, 1, 4, 1)
+GEMM_TILES(16, 128, 1, 8, 1)
+GEMM_TILES(32, 128, 2, 8, 1)
+GEMM_TILES(48, 128, 3, 8, 1)
+GEMM_TILES(80, 128, 5, 8, 1)
+GEMM_TILES(32, 256, 2, 8, 2)
+GEMM_TILES(48, 256, 3, 8, 2)
+GEMM_TILES(64, 256, 4, 8, 2)
+#undef GEMM_TILES
+
+// The manifest op's launch at up to 64 rows: the 32 x 128 tile, under one name per K = 1024 * KTW that the op has
+// it for (the K still comes as an argument: fixed at compile time, the hoisted request offsets spilled).
+#define GEMM_SMALL(KTW)                                                                                        \
+  extern "C" __global__ __launch_bounds__(512) void kern_mx_gemm_bf16_s##KTW(                                   \
+      const uint8_t* w, const uint8_t* wsf, const uint8_t* xq, const uint8_t* xsf, uint16_t* y, float* dbg,    \
+      int M, int N, int K) {                                                                                   \
+    gemm_tiles<MODE_DENSE_BF16, 2, 8, 1>(w, wsf, xq, xsf, y, nullptr, dbg, M, N, K);                  \
+  }
+GEMM_SMALL(1)
+GEMM_SMALL(2)
+GEMM_SMALL(4)
+GEMM_SMALL(7)
+GEMM_SMALL(8)
+#undef GEMM_SMALL
 
 // ====================================================================================== MXFP8 x MXFP8 GEMM
 // extern:cublaslt_mxfp8_tn (crates/kern-runtime/src/cublas.rs:387-400): row-major C[m][n] (bf16, row stride

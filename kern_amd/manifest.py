@@ -200,7 +200,7 @@ def cublaslt_mxfp8_tn(n: int, rows_var: str = "tokens") -> dict:
 # var always matches the kernel's own count. The reference has no such ops (its dense MX GEMM is the
 # runtime's built-in `extern:cublaslt_mxfp8_tn`).
 GEMV_FIXED_NKT = (2, 4, 8, 14, 16)  # K / 512 with an unrolled kern_mx_gemv_bf16_r{K/512}
-WALK_KTW = (1, 2, 4, 7, 8)          # K / 1024 with a persistent kern_mx_gemv_bf16_p* / kern_mx_gemm_bf16_s*
+WALK_KTW = (1, 2, 4, 7, 8)          # K / 1024 with a persistent kern_mx_gemv_bf16_p* (and a kern_mx_gemm_bf16_s*)
 GEMV_MAX_ROWS = 16
 
 
@@ -262,8 +262,9 @@ def mxfp4_gemv_bf16(N: int, K: int, rows_var: str = "tokens") -> dict:
 def mxfp4_gemm_bf16(N: int, K: int, rows_var: str = "tokens") -> dict:
     """The dense MXFP4 x MXFP8 GEMM with bf16 out (C ABI kern_mxfp4_gemm_bf16): in u8 a [N][K/2], sf_a (the
     repacked weights), b [M][K] and sf_b (MXFP8 activations, linear scales), out bf16 c [M][N]; M = the value
-    of `rows_var`. Up to 64 rows the persistent walk over the weights (K = 1024 * {1, 2, 4, 7, 8}), else
-    the tiled GEMM, grid [N/256, ceil(M/128)]; both with a null f32 debug pointer."""
+    of `rows_var`. Up to 64 rows the 32 x 128 tiles (K = 1024 * {1, 2, 4, 7, 8}), else the ring's 128 x 256 ones,
+    grid [N/256, ceil(M/128)]; both with a null f32 debug pointer. The C ABI chooses among more tile shapes; every
+    kernel of the family accumulates K in the same order, so the bits are the same."""
     assert N % 256 == 0 and K % 512 == 0
     p = ["in buffer<u8>"] * 4 + ["out buffer<bf16>"]
     tiled = {"module": MODULE, "entry": "kern_mx_gemm_bf16", "params": p + ["bytes<4>", "i32", "i32", "i64"],
@@ -271,20 +272,18 @@ def mxfp4_gemm_bf16(N: int, K: int, rows_var: str = "tokens") -> dict:
              "args": [{"param": i} for i in range(5)] + [_rows(rows_var), {"i32": N}, {"i32": K}, {"i64": 0}]}
     if not (K % 1024 == 0 and K // 1024 in WALK_KTW):
         return {"params": p, "impl": {"launches": [tiled]}}
-    H = N // 8
-    hb = min(9, _ceil(H, 256))
-    walk = {"module": MODULE, "entry": f"kern_mx_gemm_bf16_s{K // 1024}",
-            "params": p + ["i64", "bytes<4>", "i32", "i32", "i32"], "block": [512, 1, 1], "grid": [_ceil(H, hb), 1, 1],
-            "when": {"var": rows_var, "max": 64},
-            "args": [{"param": i} for i in range(5)] + [{"i64": 0}, _rows(rows_var), {"i32": N}, {"i32": K},
-                                                        {"i32": hb}]}
-    return {"params": p, "impl": {"launches": [walk, {**tiled, "when": {"var": rows_var, "min": 65}}]}}
+    small = {"module": MODULE, "entry": f"kern_mx_gemm_bf16_s{K // 1024}",
+             "params": p + ["i64", "bytes<4>", "i32", "i32"], "block": [512, 1, 1],
+             "grid": [N // 128, {"ceil_div": [rows_var, 32]}, 1], "when": {"var": rows_var, "max": 64},
+             "shared_mem": 4 * 16384 + _ceil(32 * (K // 512 + 1), 64) * 1024,  # kSmallTiles' {32, 128} (capi.cpp)
+             "args": [{"param": i} for i in range(5)] + [{"i64": 0}, _rows(rows_var), {"i32": N}, {"i32": K}]}
+    return {"params": p, "impl": {"launches": [small, {**tiled, "when": {"var": rows_var, "min": 65}}]}}
 
 
 def mxfp4_gemm_e4m3(N: int, K: int, rows_var: str = "tokens") -> dict:
     """The dense MXFP4 x MXFP8 GEMM with per-tensor e4m3 out (C ABI kern_mxfp4_gemm_e4m3, config 3's prefill
     GEMM): in u8 a [N][K/2], sf_a (repacked weights), b [M][K], sf_b (MXFP8 activations), out u8 c [M][N] =
-    e4m3(acc * d_scale[0]), in f32 d_scale [1]; M = the value of `rows_var`. One tiled launch, grid
+    e4m3(acc * d_scale[0]), in f32 d_scale [1]; M = the value of `rows_var`. One launch of the ring, grid
     [N/256, ceil(M/128)], with a null f32 debug pointer."""
     assert N % 256 == 0 and K % 512 == 0
     p = ["in buffer<u8>"] * 4 + ["out buffer<u8>", "in buffer<f32>"]

@@ -461,3 +461,35 @@ def test_ring_epilogue_stores_are_never_lane_conditional(fn):
         j = at[a + 4 + 4 * off]
         skipped = [ins[s][1] for s in stores if i < s < j]
         assert not skipped, f"{fn}: s_cbranch_execz at {a:#x} jumps over {skipped}"
+
+
+@pytest.mark.parametrize("tile,nx,nf,stages", [("t16x32", 4, 1, 8), ("t16x64", 2, 1, 8), ("t16x128", 1, 1, 4),
+                                               ("t32x128", 2, 1, 4), ("t48x128", 3, 1, 4), ("t80x128", 5, 1, 3),
+                                               ("t32x256", 2, 2, 3), ("t48x256", 3, 2, 3), ("t64x256", 4, 2, 3)])
+@pytest.mark.parametrize("out", ["bf16", "e4m3"])
+def test_small_tile_requests_are_as_counted(out, tile, nx, nf, stages):
+    """The small tiles wait for a stage's activations by counting the requests sent after them: 5 * nf weight and
+    scale loads and nx buffer->LDS requests a step. In the built code object every step of the loop sends exactly
+    those between its barrier and the next one's, the last round only its first step's nx, and each barrier follows
+    a wait no looser than the count."""
+    import re
+
+    ins = _disassembly(f"kern_mx_gemm_{out}_{tile}")
+    segs, waits, cur, wait = [], [], [0, 0], 63
+    for _, op, arg in ins:
+        if op == "s_barrier":
+            segs.append(cur), waits.append(wait)
+            cur, wait = [0, 0], 63
+        elif op.startswith("buffer_load"):
+            cur[1 if arg.endswith("lds") else 0] += 1
+        elif op == "s_waitcnt" and "vmcnt" in arg:
+            wait = int(re.search(r"vmcnt\((\d+)\)", arg).group(1))
+    segs.append(cur)
+    nw = 5 * nf
+    assert len(waits) == 2 * stages
+    assert segs[0][0] == stages * nw and segs[0][1] >= (stages - 1) * nx + 1  # the prologue, after the token scales
+    assert segs[1:stages + 1] == [[nw, nx]] * stages
+    assert segs[stages + 1:] == [[0, nx]] + [[0, 0]] * (stages - 1)
+    full = (stages - 1) * nw + (stages - 2) * nx
+    want = [full] * (stages + 1) + [(stages - 1 - i) * (nw + nx) for i in range(1, stages)]
+    assert all(w <= x for w, x in zip(waits, want)), (waits, want)
