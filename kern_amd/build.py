@@ -86,6 +86,9 @@ ENTRIES = {
     "kern_iota_i32": ["out buffer<i32>", "i32", "i32", "i32", "i32"],
     "kern_mx_gemm_mxfp8": ["in buffer<fp8e4m3>", "in buffer<fp8e4m3>", "out buffer<bf16>", "in buffer<u8>",
                            "in buffer<u8>", "i32", "i32", "i32", "i32"],
+    **{f"kern_mx_gemm_mxfp8_t{t}": ["in buffer<fp8e4m3>", "in buffer<fp8e4m3>", "out buffer<bf16>", "in buffer<u8>",
+                                    "in buffer<u8>", "i32", "i32", "i32", "i32"]
+       for t in ("16x16", "16x32", "16x64", "32x64", "32x128", "48x64", "64x64")},
 }
 
 

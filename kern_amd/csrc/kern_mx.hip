@@ -2158,6 +2158,222 @@ extern "C" __global__ __launch_bounds__(512) void kern_mx_gemm_mxfp8(const uint8
   }
 }
 
+// ------------------------------------------- MXFP8 x MXFP8 of small and middle batches: K split over the waves
+// kern_mx_gemm_mxfp8 gives M <= 128 one workgroup per 256 weight rows (36 at N = 9216) and waits a barrier per k-tile.
+// gemm8_tiles takes tiles of 16*MT token rows x 16*NG weight rows, one workgroup each, whose eight waves take every
+// eighth k-tile for the whole tile, so no operand byte is requested twice by a workgroup, no barrier comes before the
+// end, and a wave reads each operand fragment from LDS once for MT or NG multiplies:
+//   * weights are requested row-contiguous (8 rows of 128 bytes a request) into registers, one k-tile ahead, group by
+//     group, and pass through 4 KiB of the wave's LDS into operand pieces. Requested straight in operand pieces
+//     (16 rows' half lines a request) the kernel took 37 us at M = 72, N = 9216, K = 7168 against 24 (with N split
+//     over the waves); with both operands in an LDS ring there is room for two stages: 23;
+//   * activations go through two k-tiles of the wave's LDS by buffer->LDS requests;
+//   * scales: the 16 bytes at (r % 32) * 16 of a 128-row block's 512 are the dwords of rows r % 32 + 32 i, so two
+//     requests bring a tile's weight scales (a dword request per 16 rows: 21.4 against 17.5 us).
+// The partial sums of the eight waves meet in LDS, in wave order. A CU then takes in about 37 B a clock, as in
+// gemm_tiles. Against kern_mx_gemm_mxfp8 (graph replays, three copies in turn, us): M = 72, N = 9216, K = 7168 55.4 ->
+// 17.3; M = 72, N = 2048, K = 7168 55 -> 10; M = 16, N = 4096, K = 2048 17.9 -> 3.2; M = 200, N = 4096, K = 7168
+// 57.8 -> 16.1; M = 500, N = 4096, K = 2048 22.0 -> 13.4.
+template <int MT, int NG>
+struct Tile8Cfg {
+  static constexpr int NX = 2 * MT;                  // activation requests of a k-tile
+  static constexpr int XB = MT * 2048;               // one k-tile of the tile's token rows
+  static_assert(MT * NG <= 16 && 4 * NG + NX <= 63, "the waves' sums take at most 128 KiB; the waits are vmcnts");
+};
+
+template <int MT, int NG>
+KERN_DEV void gemm8_tiles(const uint8_t* __restrict__ xq, const uint8_t* __restrict__ w, uint16_t* __restrict__ y,
+                          const uint8_t* __restrict__ xsf, const uint8_t* __restrict__ wsf, int M, int N, int K,
+                          int ldc) {
+  using C = Tile8Cfg<MT, NG>;
+  constexpr int TM = 16 * MT, TN = 16 * NG, NX = C::NX;
+  extern __shared__ __attribute__((aligned(1024))) uint8_t tile_lds[];  // per wave: two k-tiles of X, 4 KiB for W
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, q = lane >> 4;
+  const int KT = (K + 127) >> 7, KB = K >> 5;
+  const int total = gridDim.x * gridDim.y, lin = blockIdx.x + gridDim.x * blockIdx.y, xcd = lin & 7;
+  const int tile = xcd * (total >> 3) + min(xcd, total & 7) + (lin >> 3);
+  const int nt = tile / (int)gridDim.y, mt = tile - nt * (int)gridDim.y;
+  const int m0 = mt * TM, rows = min(TM, M - m0);
+  const int n0 = nt * TN, cols = min(TN, N - n0);
+  const int n = (KT - wave + 7) >> 3;  // this wave's k-tiles: wave, wave + 8, ..
+  const __amdgpu_buffer_rsrc_t xr =
+      __builtin_amdgcn_make_buffer_rsrc((void*)(xq + (int64_t)m0 * K), (short)0, rows * K, 0x00020000);
+  const __amdgpu_buffer_rsrc_t wr =
+      __builtin_amdgcn_make_buffer_rsrc((void*)(w + (int64_t)n0 * K), (short)0, cols * K, 0x00020000);
+  const __amdgpu_buffer_rsrc_t xsr =
+      __builtin_amdgcn_make_buffer_rsrc((void*)xsf, (short)0, ((M + 127) >> 7) * KT * 512, 0x00020000);
+  const __amdgpu_buffer_rsrc_t wsr =
+      __builtin_amdgcn_make_buffer_rsrc((void*)wsf, (short)0, ((N + 127) >> 7) * KT * 512, 0x00020000);
+  // a request moves 8 rows, 16 bytes a lane: the lane's chunk of the k-tile by the parity of the row block, swizzled
+  // as the ring's; rows past the operand lie past the resource's end
+  int kc[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) kc[i] = ((lane & 7) ^ ((4 * i + (lane >> 4)) & 7)) << 4;
+  int xo[NX], wo[2 * NG];
+#pragma unroll
+  for (int i = 0; i < NX; ++i) {
+    const int row = 8 * i + (lane >> 3);
+    xo[i] = row < rows ? row * K + kc[i & 1] : 0x7fff0000;
+  }
+#pragma unroll
+  for (int i = 0; i < 2 * NG; ++i) {
+    const int row = 8 * i + (lane >> 3);
+    wo[i] = row < cols ? row * K + kc[i & 1] : 0x7fff0000;
+  }
+  auto sf_off = [&](int r) { return (r >> 7) * KT * 512 + (r & 31) * 16 + ((r & 127) >> 5) * 4; };
+  int xso[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) xso[t] = 16 * t + c < rows ? sf_off(m0 + 16 * t + c) : 0x7fff0000;
+  // the tile's weight rows lie in one 128-row block: its 16 bytes at (r % 32) * 16 are the dwords of rows r % 32 + 32 i
+  const int wsb = (n0 >> 7) * KT * 512 + c * 16, wi0 = (n0 & 127) >> 5;
+  // this wave's LDS: two k-tiles of token rows, two 16-row weight groups
+  uint8_t* xst = tile_lds + wave * (2 * C::XB + 4096);
+  uint8_t* wst = xst + 2 * C::XB;
+  auto dma = [&](int i) {
+    const int k0 = (wave + 8 * i) * 128;
+    uint8_t* st = xst + (i & 1) * C::XB;
+#pragma unroll
+    for (int p = 0; p < NX; ++p) {
+      const int o = k0 + kc[p & 1] < K ? xo[p] + k0 : 0x7fff0000;  // chunks past K: zeros
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void_t*)(st + p * 1024), 16, o, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  v4u wv[2 * NG];
+  uint32_t sx[MT];
+  v4u sw[2];
+  auto load_w = [&](int i, int g) {
+    const int k0 = (wave + 8 * i) * 128;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int o = k0 + kc[e] < K ? wo[2 * g + e] + k0 : 0x7fff0000;
+      wv[2 * g + e] = __builtin_amdgcn_raw_buffer_load_b128(wr, o, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  auto load_s = [&](int i) {
+    const int so = __builtin_amdgcn_readfirstlane((wave + 8 * i) * 512);
+#pragma unroll
+    for (int t = 0; t < MT; ++t) sx[t] = __builtin_amdgcn_raw_buffer_load_b32(xsr, xso[t], so, 0);
+#pragma unroll
+    for (int e = 0; e < (NG > 1 ? 2 : 1); ++e) sw[e] = __builtin_amdgcn_raw_buffer_load_b128(wsr, wsb + 256 * e + (NG == 1 ? (n0 & 16) * 16 : 0), so, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  v4f acc[MT][NG];
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int g = 0; g < NG; ++g) acc[t][g] = (v4f){0.f, 0.f, 0.f, 0.f};
+  auto body = [&](int i, auto LASTc) {
+    constexpr bool LAST = decltype(LASTc)::value;
+    // X(i) has landed once only the requests after it are in flight: X(i + 1) and two k-tiles of W (one at i = 0)
+    if (LAST) {
+      if (i == 0)
+        WAIT_VMCNT(2 * NG);
+      else
+        WAIT_VMCNT(4 * NG);
+    } else {
+      if (i == 0)
+        WAIT_VMCNT(2 * NG + NX);
+      else
+        WAIT_VMCNT(4 * NG + NX);
+    }
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    const int kt = wave + 8 * i;
+    const uint8_t* st = xst + (i & 1) * C::XB;
+    const bool vs = 4 * kt + q < KB;  // this lane's k block lies within K (else its scale is read as 1.0)
+    v8i xb[MT];
+    int sxv[MT], swv[NG];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      const int row = 16 * t + c, z = (row >> 1) & 7;
+      const v4i lo = *reinterpret_cast<const v4i*>(st + row * 128 + ((q ^ z) << 4));
+      const v4i hi = *reinterpret_cast<const v4i*>(st + row * 128 + (((q + 4) ^ z) << 4));
+      xb[t] = (v8i){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    }
+    WAIT_LGKMCNT0;  // read before the slot's refill is requested
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    if (!LAST && i + 2 < n) dma(i + 2);
+#pragma unroll
+    for (int t = 0; t < MT; ++t) sxv[t] = vs ? (int)(sx[t] >> (8 * q)) : 127;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      const v4u d4 = sw[g & 1];
+      const int i4 = wi0 + (g >> 1);
+      const uint32_t d = NG == 8 ? d4[(g >> 1) & 3] : (i4 == 0 ? d4[0] : i4 == 1 ? d4[1] : i4 == 2 ? d4[2] : d4[3]);
+      swv[g] = vs ? (int)(d >> (8 * q)) : 127;
+    }
+    if (!LAST) load_s(i + 1);
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      uint8_t* ws = wst + (g & 1) * 2048;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) *reinterpret_cast<v4u*>(ws + e * 1024 + lane * 16) = wv[2 * g + e];
+      if (!LAST) load_w(i + 1, g);
+      WAVE_LDS_SYNC();
+      const int zc = (c >> 1) & 7;
+      const v4i a0 = *reinterpret_cast<const v4i*>(ws + c * 128 + ((q ^ zc) << 4));
+      const v4i a1 = *reinterpret_cast<const v4i*>(ws + c * 128 + (((q + 4) ^ zc) << 4));
+      WAVE_LDS_SYNC();
+      const v8i a = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+        acc[t][g] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, xb[t], acc[t][g], 0, 0, 0, swv[g], 0, sxv[t]);
+    }
+  };
+  if (n > 0) {
+    load_s(0);
+    dma(0);
+    if (n > 1) dma(1);
+#pragma unroll
+    for (int g = 0; g < NG; ++g) load_w(0, g);
+    int i = 0;
+    for (; i + 1 < n; ++i) body(i, IC<0>{});
+    body(i, IC<1>{});
+  }
+  // the waves' partial sums, over the same LDS once every wave is done with it (its last requests were waited for)
+  v4f* red = reinterpret_cast<v4f*>(tile_lds);
+  __syncthreads();
+#pragma unroll
+  for (int p = 0; p < MT * NG; ++p) red[(wave * MT * NG + p) * 64 + lane] = acc[p / NG][p % NG];
+  __syncthreads();
+  for (int p = wave; p < MT * NG; p += 8) {
+    v4f s = red[p * 64 + lane];
+#pragma unroll
+    for (int k = 1; k < 8; ++k) s += red[(k * MT * NG + p) * 64 + lane];
+    const int t = p / NG, g = p - t * NG, col = n0 + 16 * g + 4 * q, row = 16 * t + c;
+    if (row >= rows || col >= N) continue;
+    uint16_t* dst = y + (int64_t)(m0 + row) * ldc + col;
+    if (col + 3 < N && ((((uintptr_t)dst) & 7) == 0)) {
+      *reinterpret_cast<uint2*>(dst) = make_uint2(bf16x2_hw(s[0], s[1]), bf16x2_hw(s[2], s[3]));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (col + e < N) dst[e] = (uint16_t)f32_to_bf16_bits(s[e]);
+    }
+  }
+}
+
+// Entries: tile 16*MT x 16*NG as t{rows}x{weights}, grid [ceil(N / weights), ceil(M / rows)], block 512, dynamic LDS the
+// larger of 8 * (MT + 1) * 4 KiB (the waves' stages) and 8 * MT * NG KiB (their sums).
+#define GEMM8_TILES(TM, TN, MT, NG)                                                                            \
+  extern "C" __global__ __launch_bounds__(512) void kern_mx_gemm_mxfp8_t##TM##x##TN(                            \
+      const uint8_t* a, const uint8_t* w, uint16_t* c, const uint8_t* a_sf, const uint8_t* w_sf, int M, int N, \
+      int K, int ldc) {                                                                                        \
+    gemm8_tiles<MT, NG>(a, w, c, a_sf, w_sf, M, N, K, ldc);                                                    \
+  }
+GEMM8_TILES(16, 16, 1, 1)
+GEMM8_TILES(16, 32, 1, 2)
+GEMM8_TILES(16, 64, 1, 4)
+GEMM8_TILES(32, 64, 2, 4)
+GEMM8_TILES(32, 128, 2, 8)
+GEMM8_TILES(48, 64, 3, 4)
+GEMM8_TILES(64, 64, 4, 4)
+#undef GEMM8_TILES
+
 // ====================================================================================== routing
 // op moe_routing (head.json:25117): in i32 topk_idx[T][topk]; out counts [2E], cta_batch, cta_limit,
 // num_non_exiting[1], total_padded[1], route_map, exp2perm [T*topk]; launch adds i32 T, i32 topk,

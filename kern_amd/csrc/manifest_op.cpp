@@ -320,6 +320,7 @@ const BlockRule kBlockRules[] = {
     {"kern_mx_gemm_bf16_t16x32", false, 128, false}, {"kern_mx_gemm_e4m3_t16x32", false, 128, false},
     {"kern_mx_gemm_bf16_t16x64", false, 256, false}, {"kern_mx_gemm_e4m3_t16x64", false, 256, false},
     {"kern_mx_gemm_e4m3", false, 512, false},       {"kern_mx_gemm_mxfp8", false, 512, false},
+    {"kern_mx_gemm_mxfp8_t", true, 512, false},
     {"kern_mx_bmm_fc1", false, 512, false},         {"kern_mx_bmm_fc2", false, 512, false},
     {"kern_mx_routing", false, 1024, false},        {"kern_mx_routing_count", false, 1024, false},
     {"kern_mx_routing_scan", false, 1024, false},   {"kern_mx_routing_rank", false, 1024, false},

@@ -1,17 +1,17 @@
-"""The dense GEMM's small tiles (kern_mx_gemm_{bf16,e4m3}_t{rows}x{weights}) against the ring's 128 x 256 kernel, bit
-for bit (every kernel of the family accumulates K in the same order), and the rule that picks one.
+"""The dense GEMMs' small tiles: the MXFP4 ones (kern_mx_gemm_{bf16,e4m3}_t{rows}x{weights}) against the ring's
+128 x 256 kernel, bit for bit (every kernel of the family accumulates K in the same order), the MXFP8 ones
+(kern_mx_gemm_mxfp8_t{rows}x{weights}) against the oracle, and the rules that pick one.
 
 Each tile runs at its edges: one row, one row short of a whole tile, one past it; K from one k group of 512 to past two
 rounds of its stages, every remainder among them; fewer and more tiles than the eight XCDs. The ring kernel is compared
 with the CPU oracle in test_gpu_stack.py and test_gpu_sweep.py; here the entry as the C ABI picks it is as well, on both
 sides of a switch and where it takes the ring for some rows and small tiles for the rest.
 """
-import os
-
+import numpy as np
 import pytest
 
 from kern_amd import workload as wl
-from tests._util import assert_gemm_close, bf16_to_f32, to_dev, to_np
+from tests._util import assert_gemm_close, bf16_to_f32, r128c4_offsets, to_dev, to_np
 
 pytestmark = pytest.mark.gpu
 
@@ -78,3 +78,32 @@ def test_dense_gemm_as_picked(ops, oracle, M, N, K):
     torch.cuda.synchronize()
     _, acc = oracle.gemm_e4m3_pt(to_np(w), to_np(s), to_np(q), to_np(qs), N, K, 1.0)
     assert_gemm_close(bf16_to_f32(to_np(c)), acc, "dense")
+
+
+def _mxfp8(ops, rows, K, seed):
+    """MXFP8 rows as quantized on the device, scales tiled 128x4 with NaN codes in the padding."""
+    q, sf = ops.quantize_mxfp8(to_dev(wl.activations_bf16(seed, rows, K, outlier_frac=0.01)))
+    t = np.full(ops.r128c4_bytes(rows, K // 32), 255, np.uint8)
+    t[r128c4_offsets(rows, K // 32)] = to_np(sf)
+    return to_np(q), t
+
+
+@pytest.mark.parametrize("rows,weights", [(16, 16), (16, 32), (16, 64), (32, 64), (32, 128), (48, 64), (64, 64)])
+def test_mxfp8_tiles(ops, oracle, rows, weights):
+    """K from one 32-wide block to past two k-tiles a wave (8 waves take every eighth 128-wide k-tile), partial last
+    k-tiles; rows one short of and one past whole tiles and across a 128-row scale block; n and ldc odd."""
+    mod = ops.Module(ops.HSACO_PATH)
+    for M, N, K in [(1, 1, 32), (rows, weights, 128), (rows - 1, weights + 1, 1000 // 32 * 32), (3 * rows + 1, 263, 1120),
+                    (130, 200, 2112), (rows + 1, 2 * weights - 3, 3200)]:
+        print(f"[tile8] {rows}x{weights} M={M} N={N} K={K}", flush=True)
+        (qa, ta), (qw, tw) = _mxfp8(ops, M, K, 80), _mxfp8(ops, N, K, 81)
+        ldc = N + 3
+        out = torch.full((M + 1, ldc), 7.0, dtype=torch.bfloat16, device="cuda")
+        mt, ng = rows // 16, weights // 16
+        mod.launch(f"kern_mx_gemm_mxfp8_t{rows}x{weights}", (-(-N // weights), -(-M // rows)), (512,), to_dev(qa), to_dev(qw),
+                   out, to_dev(ta), to_dev(tw), M, N, K, ldc, shared=max(32768 * (mt + 1), 8192 * mt * ng))
+        torch.cuda.synchronize()
+        got = bf16_to_f32(to_np(out))
+        assert (got[:, N:] == 7.0).all() and (got[M] == 7.0).all()
+        assert_gemm_close(got[:M, :N], oracle.mxfp8_gemm(qa, qw, ta, tw, M, N, K), f"{rows}x{weights} {M}x{N}x{K}")
+    mod.close()
