@@ -609,45 +609,45 @@ extern "C" int kern_mxfp4_gemv_bf16(const void* x, const void* w, const void* w_
   REQUIRE(M >= 1 && M <= 16 && N > 0 && N % 16 == 0 && K > 0 && K % 512 == 0 && K <= 16384,
           "mxfp4_gemv_bf16: need 1 <= M <= 16, N %% 16 == 0, K %% 512 == 0, K <= 16384 (M=%d N=%d K=%d)", M, N, K);
   REQUIRE(x && w && w_sf && y, "mxfp4_gemv_bf16: null buffer");
-  const int32_t kg = K / 512;
-  // K = 512 * NKT with an unrolled instance for NKT: each of the four waves owns NKT consecutive k-tiles
-  const char* fixed = kg == 2 ? "kern_mx_gemv_bf16_r2" : kg == 4 ? "kern_mx_gemv_bf16_r4" : kg == 8 ? "kern_mx_gemv_bf16_r8"
-                      : kg == 14 ? "kern_mx_gemv_bf16_r14" : kg == 16 ? "kern_mx_gemv_bf16_r16" : nullptr;
-  // Also taken at M = 3, and at any M while N <= 8192, as long as the x slices fit in 144 KiB of LDS.
-  // Each workgroup reads all of x, so the persistent kernel's x reuse wins from M = 4 on at large N
-  // (K = 7168, N = 9216: 9.8 against 10.1 us; N = 18432: 13.2 against 16.3). At M = 3 the two are within
-  // 5% either way (N = 9216: 9.2 against 9.7 us; N = 18432: 13.6 against 13.2). At N <= 8192 the
-  // persistent workgroups own four or fewer half groups, and the row-group kernel stays ahead:
-  //   N = 7168, K = 8192, M = 8: 10.0 against 10.5 us;
-  //   N = 4096, K = 4096, M = 16: 5.3 against 7.5 us.
-  if (fixed && 2 * M * K <= 144 * 1024 && (M <= 3 || N <= 8192)) {
-    // one workgroup per 16-row group; each wave's x slice (M * NKT * 256 B) in its own LDS region
+  const int32_t kg = K / 512, lds_x = 2 * M * K;
+  char entry[40];
+  // Row groups (r{K/512}: one workgroup per 16 weight rows, each reading all of x) against the persistent walk
+  // (p{..}: x read once per workgroup, of which there are about 256), by a sweep of both over 8559 launches (M = 1..16,
+  // N = 1024..18432, every K up to 8192, graph replays): the rule is within 1% of the faster one on average.
+  //   M <= 3: row groups at any N (M = 1, N = 2048: 0.71 of the walk's time, N = 18432: 0.94; M = 3 at N > 8192 the
+  //   two are within 5%).
+  //   M > 3: row groups while they all run at once, N <= 4096 per workgroup of their x that a CU's LDS holds, at most
+  //   two (M = 5, N = 3584, K = 7680: 5.4 against 7.7 us), else the walk (M = 8, N = 7168, K = 7680: 9.2 against
+  //   10.1 us; M = 16, N = 8192, K = 2560: 5.8 against 8.5). At K = 512 the walk is ahead from N = 4096 on (M = 16,
+  //   N = 7168: 3.4 against 3.9 us).
+  const bool one_round = N <= 4096 * std::min(2, 163840 / (lds_x + 5120)) && (kg > 1 || N <= 4096);
+  if (kg <= 16 && lds_x <= 144 * 1024 && (M <= 3 || one_round)) {
+    // each wave's x slice (M * K / 2 bytes) in its own LDS region
     Args a;
     a.put(x), a.put(w), a.put(w_sf), a.put(y), a.put(M), a.put(N), a.put(K);
-    return launch(fixed, (uint32_t)(N / 16), 1, 1, 256, stream, a, 2u * (uint32_t)M * (uint32_t)K);
+    snprintf(entry, sizeof entry, "kern_mx_gemv_bf16_r%d", kg);
+    return launch(entry, (uint32_t)(N / 16), 1, 1, 256, stream, a, (uint32_t)lds_x);
   }
   if (M <= 2) {
-    // other K: the same, each wave owning whole 512-wide k groups (a floor or ceiling of KG/4) in a loop,
+    // K > 8192: the same, each wave owning whole 512-wide k groups (a floor or ceiling of KG/4) in a loop,
     // and keeping their x (1 KiB per token and group) in its own LDS region
     const int32_t gmax = (kg + 3) / 4;
     Args a;
     a.put(x), a.put(w), a.put(w_sf), a.put(y), a.put(M), a.put(N), a.put(K), a.put(gmax);
     return launch("kern_mx_gemv_bf16_rg", (uint32_t)(N / 16), 1, 1, 256, stream, a, 4u * (uint32_t)(gmax * M) * 1024u);
   }
-  static const char* const persistent[9] = {nullptr, "kern_mx_gemv_bf16_p1", "kern_mx_gemv_bf16_p2", nullptr,
-                                            "kern_mx_gemv_bf16_p4", nullptr, nullptr, "kern_mx_gemv_bf16_p7",
-                                            "kern_mx_gemv_bf16_p8"};
-  if (K % 1024 == 0 && K / 1024 <= 8 && persistent[K / 1024]) {
-    // about 256 workgroups of 8 waves, each owning hb <= 9 half groups of 8 rows (at most five 16-row
-    // groups); wave w owns k-tiles [w*K/1024, (w+1)*K/1024) and holds their x in registers, one k-tile
-    // at a time, passed through 4 KiB of LDS of its own
+  if (kg <= 16) {
+    // about 256 workgroups of 8 waves, each owning hb <= 9 half groups of 8 rows (at most five 16-row groups); a
+    // wave owns a run of K/1024 k-tiles (rounded down or up where K is an odd multiple of 512: p{..}h) and holds
+    // their x in registers, one k-tile at a time, passed through 4 KiB of LDS of its own
     const int32_t H = N / 8;
     const int32_t hb = std::min<int32_t>(9, (H + 255) / 256);
     Args a;
     a.put(x), a.put(w), a.put(w_sf), a.put(y), a.put(M), a.put(N), a.put(K), a.put(hb);
-    return launch(persistent[K / 1024], (uint32_t)((H + hb - 1) / hb), 1, 1, 512, stream, a);
+    snprintf(entry, sizeof entry, "kern_mx_gemv_bf16_p%d%s", (kg + 1) / 2, kg % 2 ? "h" : "");
+    return launch(entry, (uint32_t)((H + hb - 1) / hb), 1, 1, 512, stream, a);
   }
-  // any other shape: one workgroup per row group, x staged per workgroup in slices
+  // K > 8192 at M > 2: one workgroup per row group, x staged per workgroup in slices
   // sb: k-tiles per wave whose slice of x is staged in LDS at once (at most four 16-byte pieces per lane,
   // M * sb <= 16, sb divides K/512); nb: k-tiles per wave whose weights are in flight together (the
   // largest of the kernel's batch sizes dividing sb)

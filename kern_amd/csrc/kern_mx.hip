@@ -148,8 +148,9 @@ typedef __attribute__((address_space(1))) void glob_void_t;
 // non-gated) [N][K/2], in u8 w_sf (repacked), out bf16 y[M][N], i32 M, launch i32 N, i32 K, i32 nb, i32 sb.
 // Grid N/16, block 256, dynamic LDS M*(sb*1024 + 16) + K/2 bytes: one 16-row group per workgroup. Wave w
 // takes the 128-wide k-tiles kt = 4i + w (equal shares; its scale is byte w of each scale dword of the
-// group). x is consumed in slices of sb k-tiles per wave (sb divides K/512, M*sb <= 16), weights in rounds
-// of nb fragments per wave (nb divides sb). Each slice of x, and with the first slice the row group's
+// group). Taken for K > 8192 at M > 2. x is consumed in slices of sb k-tiles per wave (sb divides K/512,
+// M*sb <= 16), weights in rounds of nb fragments per wave (nb divides sb). Each slice of x, and with the
+// first slice the row group's
 // whole scale block, goes from memory straight into LDS (buffer loads to LDS, no registers); the round's
 // weight fragments are requested behind them in straight-line code, so waiting for the LDS data leaves
 // the weights in flight, and each fragment is multiplied as soon as it lands. At M = 1, K = 7168 one
@@ -274,7 +275,7 @@ extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
   }
 }
 
-// ---------------------------------------------------------------- decode GEMV, M <= 2: one row group per workgroup
+// ---------------------------------------------------------------- decode GEMV, M <= 2, K > 8192: a row group a workgroup
 // Same operand mapping as above (fp4 rows decoded by V_CVT_SCALEF32_PK_BF16_FP4 into the A operand of
 // V_MFMA_F32_16X16X32_BF16, tokens in the B columns). One workgroup of four waves per 16-row group, so
 // all N/16 workgroups are resident at once (18 waves per CU at N = 18432). Wave w owns the 512-wide k
@@ -371,9 +372,11 @@ extern "C" __global__ __launch_bounds__(256) void kern_mx_gemv_bf16_rg(
 
 // --------------------------------------------- decode GEMV at fixed K: the same, fully unrolled
 // Taken (kern_mxfp4_gemv_bf16) for K = 512 * NKT while the x slices, 2*M*K bytes of dynamic LDS, fit in
-// 144 KiB, at M <= 3 or at any M <= 16 while N <= 8192; with the static ssc and red arrays (at most 5 KiB)
-// the workgroup stays below the 160 KiB of LDS.
-// For K = 512 * NKT with NKT in {2, 4, 8, 14, 16} each wave owns exactly NKT consecutive k-tiles (k-tile
+// 144 KiB, at M <= 3 or while all row groups run at once; with the static ssc and red arrays (at most 9 KiB)
+// the workgroup stays below the 160 KiB of LDS. Against the slice-staging kernel above, which every K but
+// 512 * {2, 4, 8, 14, 16} took before (a workgroup barrier per x slice of at most 16/M k-tiles): M = 5,
+// N = 3584, K = 7680 11.9 -> 5.4 us; against kern_mx_gemv_bf16_rg (M <= 2) 5% shorter on average.
+// For K = 512 * NKT, NKT = 1..16, each wave owns exactly NKT consecutive k-tiles (k-tile
 // ranges, not whole 512-wide groups) and its loop is unrolled, so the weight stream has no requests past
 // its end and no branches around them: every request is one the compiler's wait counts can see, and an
 // extra request per wave costs measurably (one unneeded 256 B scale fragment per wave: +0.8 us at N =
@@ -402,6 +405,10 @@ KERN_DEV void gemv_rows_fixed(const uint16_t* __restrict__ x, const uint8_t* __r
   const __amdgpu_buffer_rsrc_t sr =
       __builtin_amdgcn_make_buffer_rsrc((void*)(wsf + (int64_t)rg * KG * 256), (short)0, KG * 256, 0x00020000);
   if (lane < ns * 16) __builtin_amdgcn_raw_ptr_buffer_load_lds(sr, (lds_void_t*)&ssc[wave][0], 16, kgA * 256 + lane * 16, 0, 0, 2);
+  if constexpr (NSMAX > 4) {  // NKT = 15: k-tiles 15..29 touch five fragments, one past what a request holds
+    if (lane < ns * 16 - 64)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(sr, (lds_void_t*)&ssc[wave][256], 16, kgA * 256 + 1024 + lane * 16, 0, 0, 2);
+  }
   __builtin_amdgcn_sched_barrier(0);
   const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(w + ((int64_t)rg * KT + kt0) * 1024), (short)0, NKT * 1024, 0x00020000);
@@ -430,7 +437,8 @@ KERN_DEV void gemv_rows_fixed(const uint16_t* __restrict__ x, const uint8_t* __r
   for (int i = 0; i < NKT; ++i) {
     const v4u wv = buf[i % D];
     const int kt = kt0 + i;
-    const uint32_t dw = ((ph + i) >> 2) == (i >> 2) ? sdw[i >> 2] : sdw[(i >> 2) + 1];
+    // (i % 4 == 0 needs no second dword, and at NKT % 4 == 1 the last fragment has none)
+    const uint32_t dw = (i & 3) == 0 || ((ph + i) >> 2) == (i >> 2) ? sdw[i >> 2] : sdw[(i >> 2) + ((i & 3) != 0)];
     const float s = fp4_cvt_scale((dw >> (8 * (kt & 3))) & 255u);
     if (xlive) {
 #pragma unroll
@@ -468,10 +476,21 @@ KERN_DEV void gemv_rows_fixed(const uint16_t* __restrict__ x, const uint8_t* __r
       uint16_t* __restrict__ y, int M, int N, int K) {                                                         \
     gemv_rows_fixed<NKT>(x, w, wsf, y, M, N, K);                                                            \
   }
+GEMV_ROWS_FIXED(1)
 GEMV_ROWS_FIXED(2)
+GEMV_ROWS_FIXED(3)
 GEMV_ROWS_FIXED(4)
+GEMV_ROWS_FIXED(5)
+GEMV_ROWS_FIXED(6)
+GEMV_ROWS_FIXED(7)
 GEMV_ROWS_FIXED(8)
+GEMV_ROWS_FIXED(9)
+GEMV_ROWS_FIXED(10)
+GEMV_ROWS_FIXED(11)
+GEMV_ROWS_FIXED(12)
+GEMV_ROWS_FIXED(13)
 GEMV_ROWS_FIXED(14)
+GEMV_ROWS_FIXED(15)
 GEMV_ROWS_FIXED(16)
 #undef GEMV_ROWS_FIXED
 
@@ -489,7 +508,10 @@ GEMV_ROWS_FIXED(16)
 // each request gathered 16 rows' 16-byte pieces at a 64-byte stride (M = 16: 15.4 against 14.6-15.0 us
 // at N = 18432, 12.5 against 10.5 at N = 7168, K = 8192).
 // Fragments stream six ahead. The eight partial sums meet in LDS.
-template <int KTW>
+// HALF: K = 1024*KTW - 512; waves 0-3 own KTW k-tiles and waves 4-7 KTW - 1, whose last item's requests go past
+// the buffer like those of absent row groups and whose products are skipped. These lengths took the slice-staging
+// kernel before: M = 8, N = 7168, K = 7680 14.7 -> 9.2 us; M = 16, N = 8192, K = 2560 6.9 -> 5.8 us.
+template <int KTW, bool HALF>
 KERN_DEV void gemv_persistent(const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
                               const uint8_t* __restrict__ wsf, uint16_t* __restrict__ y, int M, int N, int K, int hb) {
   constexpr int NG = 5, D = 6, TOT = NG * KTW;
@@ -501,7 +523,8 @@ KERN_DEV void gemv_persistent(const uint16_t* __restrict__ x, const uint8_t* __r
   const int h0 = blockIdx.x * hb, h1 = min(h0 + hb, H);
   const int g0 = h0 >> 1, ng = ((h1 + 1) >> 1) - g0;  // row groups touched: [g0, g0 + ng), ng <= NG
   const int c = lane & 15, kq = lane >> 4, r = lane & 15;
-  const int kt0 = wave * KTW, kgA = kt0 >> 2;
+  const int kt0 = HALF ? wave * (KTW - 1) + min(wave, 4) : wave * KTW, kgA = kt0 >> 2;
+  const bool last = !HALF || wave < 4;  // this wave has a k-tile KTW - 1
   // x: lane (c, kq) holds x[c][128*kt + 32*kq .. +32] for each of its k-tiles (absent tokens: zeros)
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)x, (short)0, M * K * 2, 0x00020000);
   // request p of a k-tile loads rows 4p .. 4p+3, 16 lanes a row and 16 B a lane (row-contiguous); absent
@@ -538,7 +561,7 @@ KERN_DEV void gemv_persistent(const uint16_t* __restrict__ x, const uint8_t* __r
   // item i = j*NG + g is fragment (g0 + g, kt0 + j); rows outside the owned half groups read zeros
   auto woff = [&](int i) -> int {
     const int g = i % NG, half = (g0 + g) * 2 + (r >> 3);
-    return (g < ng && half >= h0 && half < h1) ? (g * KT + kt0 + i / NG) * 1024 + lane * 16 : 0x40000000;
+    return (g < ng && half >= h0 && half < h1 && (i / NG < KTW - 1 || last)) ? (g * KT + kt0 + i / NG) * 1024 + lane * 16 : 0x40000000;
   };
   v4u buf[D];
 #pragma unroll
@@ -568,7 +591,7 @@ KERN_DEV void gemv_persistent(const uint16_t* __restrict__ x, const uint8_t* __r
     // row groups past the workgroup's share were loaded as zeros (requests keep one fixed order); their
     // conversions and products are skipped (a uniform branch). Every share holds row group 0, and testing
     // it at compile time keeps the compiler from sinking item 0's request into the branch behind a full wait.
-    if (g == 0 || g < ng) {
+    if ((g == 0 || g < ng) && (j < KTW - 1 || last)) {
       const float s = fp4_cvt_scale((sdw[g][(kt >> 2) - kgA] >> (8 * (kt & 3))) & 0xffu);
 #pragma unroll
       for (int jj = 0; jj < 4; ++jj) {
@@ -602,17 +625,28 @@ KERN_DEV void gemv_persistent(const uint16_t* __restrict__ x, const uint8_t* __r
   }
 }
 
-#define GEMV_PERSISTENT(KTW)                                                                                   \
-  extern "C" __global__ __launch_bounds__(512) void kern_mx_gemv_bf16_p##KTW(                                   \
+#define GEMV_PERSISTENT(NAME, KTW, HALF)                                                                       \
+  extern "C" __global__ __launch_bounds__(512) void kern_mx_gemv_bf16_p##NAME(                                  \
       const uint16_t* __restrict__ x, const uint8_t* __restrict__ w, const uint8_t* __restrict__ wsf,          \
       uint16_t* __restrict__ y, int M, int N, int K, int hb) {                                                 \
-    gemv_persistent<KTW>(x, w, wsf, y, M, N, K, hb);                                                           \
+    gemv_persistent<KTW, HALF>(x, w, wsf, y, M, N, K, hb);                                                     \
   }
-GEMV_PERSISTENT(1)
-GEMV_PERSISTENT(2)
-GEMV_PERSISTENT(4)
-GEMV_PERSISTENT(7)
-GEMV_PERSISTENT(8)
+GEMV_PERSISTENT(1, 1, false)
+GEMV_PERSISTENT(1h, 1, true)
+GEMV_PERSISTENT(2, 2, false)
+GEMV_PERSISTENT(2h, 2, true)
+GEMV_PERSISTENT(3, 3, false)
+GEMV_PERSISTENT(3h, 3, true)
+GEMV_PERSISTENT(4, 4, false)
+GEMV_PERSISTENT(4h, 4, true)
+GEMV_PERSISTENT(5, 5, false)
+GEMV_PERSISTENT(5h, 5, true)
+GEMV_PERSISTENT(6, 6, false)
+GEMV_PERSISTENT(6h, 6, true)
+GEMV_PERSISTENT(7, 7, false)
+GEMV_PERSISTENT(7h, 7, true)
+GEMV_PERSISTENT(8, 8, false)
+GEMV_PERSISTENT(8h, 8, true)
 #undef GEMV_PERSISTENT
 
 // ====================================================================================== block-scaled GEMM

@@ -199,8 +199,8 @@ def cublaslt_mxfp8_tn(n: int, rows_var: str = "tokens") -> dict:
 # rows (M, tokens) reach the kernels from the var, as a 4-byte pack, so that the dynamic LDS sized from the
 # var always matches the kernel's own count. The reference has no such ops (its dense MX GEMM is the
 # runtime's built-in `extern:cublaslt_mxfp8_tn`).
-GEMV_FIXED_NKT = (2, 4, 8, 14, 16)  # K / 512 with an unrolled kern_mx_gemv_bf16_r{K/512}
-WALK_KTW = (1, 2, 4, 7, 8)          # K / 1024 with a persistent kern_mx_gemv_bf16_p* (and a kern_mx_gemm_bf16_s*)
+GEMV_MAX_NKT = 16           # K / 512 up to which kern_mx_gemv_bf16_r* and _p* have an instance
+WALK_KTW = (1, 2, 4, 7, 8)  # K / 1024 with a kern_mx_gemm_bf16_s*
 GEMV_MAX_ROWS = 16
 
 
@@ -214,7 +214,8 @@ def _gemv_launch(N: int, K: int, M: int, rows_var: str) -> dict:
     params = ["in buffer<bf16>", "in buffer<u8>", "in buffer<u8>", "out buffer<bf16>", "bytes<4>", "i32", "i32"]
     args = [{"param": i} for i in range(4)] + [_rows(rows_var), {"i32": N}, {"i32": K}]
     row_groups = [N // 16, 1, 1]
-    if kg in GEMV_FIXED_NKT and 2 * M * K <= 144 * 1024 and (M <= 3 or N <= 8192):
+    one_round = N <= 4096 * min(2, 163840 // (2 * M * K + 5120)) and (kg > 1 or N <= 4096)
+    if kg <= GEMV_MAX_NKT and 2 * M * K <= 144 * 1024 and (M <= 3 or one_round):
         # one workgroup per 16-row group, each wave's x slice (2 * M * K bytes in all) in LDS
         return {"entry": f"kern_mx_gemv_bf16_r{kg}", "params": params, "block": [256, 1, 1], "grid": row_groups,
                 "shared_mem": {"mul": [rows_var, 2 * K]}, "args": args}
@@ -223,12 +224,12 @@ def _gemv_launch(N: int, K: int, M: int, rows_var: str) -> dict:
         return {"entry": "kern_mx_gemv_bf16_rg", "params": params + ["i32"], "block": [256, 1, 1],
                 "grid": row_groups, "shared_mem": {"mul": [rows_var, 4 * gmax * 1024]},
                 "args": args + [{"i32": gmax}]}
-    if K % 1024 == 0 and K // 1024 in WALK_KTW:
+    if kg <= GEMV_MAX_NKT:
         H = N // 8
         hb = min(9, _ceil(H, 256))
-        return {"entry": f"kern_mx_gemv_bf16_p{K // 1024}", "params": params + ["i32"], "block": [512, 1, 1],
+        return {"entry": f"kern_mx_gemv_bf16_p{_ceil(kg, 2)}{'h' if kg % 2 else ''}", "params": params + ["i32"], "block": [512, 1, 1],
                 "grid": [_ceil(H, hb), 1, 1], "args": args + [{"i32": hb}]}
-    # any other shape: x staged in slices of sb k-tiles per wave, nb k-tiles of weights in flight together
+    # K > 8192: x staged in slices of sb k-tiles per wave, nb k-tiles of weights in flight together
     sb = next(c for c in range(min(kg, GEMV_MAX_ROWS // M), 0, -1) if kg % c == 0)
     nb = next((c for c in (7, 4, 2) if sb % c == 0), 1)
     return {"entry": "kern_mx_gemv_bf16", "params": params + ["i32", "i32"], "block": [256, 1, 1],

@@ -94,13 +94,13 @@ def test_repack_bitexact(ops, oracle, E, rows, K, gated):
 
 # --------------------------------------------------------------------------------------- decode GEMV
 
-# kern_mxfp4_gemv_bf16 picks a kernel by shape; the cases cover each:
-#   K = 512 * {2, 4, 8, 14, 16} with 2*M*K <= 144 KiB and M <= 3 or N <= 8192 ->
-#   kern_mx_gemv_bf16_r{2,4,8,14,16} (unrolled; M = 8 at N = 512, 16 at N = 4096, 9 at the LDS bound);
-#   M <= 2, other K -> kern_mx_gemv_bf16_rg (k groups split four ways: KG = 1, 3, 7, 32);
-#   otherwise K = 1024 * {1, 2, 4, 7, 8} -> kern_mx_gemv_bf16_p{1,2,4,7,8} (half-group shares of 1, 4,
-#   5, 6, 8 and 9, ragged last workgroups at N = 8336, 9216 and 18448, M = 10 just past the LDS bound);
-#   anything else -> kern_mx_gemv_bf16 (K = 1536, 3072).
+# kern_mxfp4_gemv_bf16 picks a kernel by shape; the cases cover each kind (test_gpu_gemv_lengths.py takes every K):
+#   K <= 8192 with 2*M*K <= 144 KiB and M <= 3, or while all row groups run at once ->
+#   kern_mx_gemv_bf16_r{K/512} (unrolled; M = 8 at N = 512, 16 at N = 4096);
+#   M <= 2, K > 8192 -> kern_mx_gemv_bf16_rg (k groups split four ways: KG = 32);
+#   otherwise K <= 8192 -> kern_mx_gemv_bf16_p{K/1024}, or p{ceil(K/1024)}h (half-group shares of 1, 4,
+#   5, 6, 8 and 9, ragged last workgroups at N = 8336, 9216 and 18448);
+#   anything else -> kern_mx_gemv_bf16.
 @pytest.mark.parametrize("M,N,K,lo,hi", [(8, 512, 1024, 124, 130), (1, 18432, 7168, 122, 132),
                                          (4, 18432, 7168, 122, 132), (16, 18432, 7168, 122, 132),
                                          (3, 1024, 2048, 100, 150),
