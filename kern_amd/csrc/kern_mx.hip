@@ -1771,7 +1771,8 @@ KERN_DEV void gemm_tiles(const uint8_t* __restrict__ w, const uint8_t* __restric
     }
     __builtin_amdgcn_sched_barrier(0);
   }
-  // buffer resources, of length zero for the steps before the first k group (zeros, no memory traffic)
+  // buffer resources, of length zero for the steps before the first k group (zeros, no memory traffic). Their scalar
+  // offset is 0 too: the range check compares the lane's offset with length - scalar offset
   const uint8_t* xb0 = xq + (int64_t)m0 * K;
   const uint8_t* wb0 = w + (int64_t)g0 * KT * 1024;
   const uint8_t* sb0 = wsf + (int64_t)g0 * KG * 256;
@@ -1783,8 +1784,8 @@ KERN_DEV void gemm_tiles(const uint8_t* __restrict__ w, const uint8_t* __restric
   int xo[NX];
 #pragma unroll
   for (int i = 0; i < NX; ++i) {
-    const int row = 8 * ((wave * NX + i) % (2 * MT)) + (lane >> 3);
-    xo[i] = row < rows ? row * K + (((lane & 7) ^ ((row >> 1) & 7)) << 4) : 0x7fffff00;
+    const int r = wave * NX + i, row = 8 * (r % (2 * MT)) + (lane >> 3);
+    xo[i] = row < rows ? row * K + r / (2 * MT) * 128 + (((lane & 7) ^ ((row >> 1) & 7)) << 4) : 0x7fffff00;
   }
   int wo[NF], so[NF];
 #pragma unroll
@@ -1795,12 +1796,12 @@ KERN_DEV void gemm_tiles(const uint8_t* __restrict__ w, const uint8_t* __restric
   }
   auto dma = [&](int v, int slot) {
     const __amdgpu_buffer_rsrc_t x_ = rsrc(xb0, rows * K, v >= p0);
-    const int kg = v - p0;
+    const int kg = max(v - p0, 0);
 #pragma unroll
     for (int i = 0; i < NX; ++i) {
       const int r = wave * NX + i;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(x_, (lds_void_t*)(tile_lds + slot * C::STAGE + r * 1024), 16, xo[i],
-                                               __builtin_amdgcn_readfirstlane((4 * kg + r / (2 * MT)) * 128), 0, 0);
+                                               __builtin_amdgcn_readfirstlane(kg * 512), 0, 0);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -1809,7 +1810,7 @@ KERN_DEV void gemm_tiles(const uint8_t* __restrict__ w, const uint8_t* __restric
   auto load_w = [&](int v, auto Ic) {
     constexpr int i = decltype(Ic)::value;
     const __amdgpu_buffer_rsrc_t w_ = rsrc(wb0, ng * KT * 1024, v >= p0), s_ = rsrc(sb0, ng * KG * 256, v >= p0);
-    const int kg = v - p0;
+    const int kg = max(v - p0, 0);
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
       ws[i][f] = __builtin_amdgcn_raw_buffer_load_b32(s_, so[f], __builtin_amdgcn_readfirstlane(kg * 256), 0);
