@@ -63,7 +63,7 @@ ENTRIES = {
        for out in ("bf16", "e4m3") for t in ("16x32", "16x64", "16x128", "32x128", "48x128", "80x128", "32x256",
                                              "48x256", "64x256")},
     **{f"kern_mx_gemm_bf16_s{ktw}": ["in buffer<u8>", "in buffer<u8>", "in buffer<u8>", "in buffer<u8>",
-                                     "out buffer<bf16>", "out buffer<f32>", "i32", "i32", "i32"]
+                                     "out buffer<bf16>", "out buffer<f32>", "i32", "i32", "i32", "i32"]
        for ktw in (1, 2, 4, 7, 8)},
     **{e: ["in buffer<i32>"] + ["out buffer<i32>"] * 7 + ["i32"] * 4
        for e in ("kern_mx_routing", "kern_mx_routing_count", "kern_mx_routing_scan", "kern_mx_routing_rank")},

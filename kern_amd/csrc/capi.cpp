@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "elf_meta.h"
+#include "pick.h"
 #include "sha256.h"
 
 #ifndef KERN_MX_SHA256
@@ -489,62 +490,7 @@ extern "C" int kern_trtllm_bmm_mxe4m3_mxe2m1_mxe4m3(const void* a_, const void* 
 
 namespace {
 
-// A dense MXFP4 x MXFP8 GEMM's kernel: one of the small tiles (kern_mx_gemm_*_t{rows}x{weights}) or the LDS ring's
-// 128 x 256 tiles. All accumulate K in the same order, so the choice does not show in the results.
-struct SmallTile {
-  int rows, weights, waves, stages;
-};
-const SmallTile kSmallTiles[] = {
-    {16, 32, 2, 8}, {16, 64, 4, 8}, {16, 128, 8, 4}, {32, 128, 8, 4}, {48, 128, 8, 4},
-    {80, 128, 8, 3}, {32, 256, 8, 3}, {48, 256, 8, 3}, {64, 256, 8, 3},
-};
-// dynamic LDS of a small tile: the activation ring, then the token scales in whole KiB
-int64_t small_tile_lds(const SmallTile& t, int64_t k) {
-  return (int64_t)t.stages * t.rows * 512 + (t.rows * (k / 512 + 1) + 63) / 64 * 1024;
-}
-// Microseconds of a launch, fitted to both kernels over 150 shapes (M = 17..3000, N = 512..9216, K = 512..8192,
-// graph replays; rms 10% for the tiles, 5% for the ring). A tile's k group costs by its token subtiles (mt), its
-// 16-row weight groups (n) and their product, its output by the product; a tile past one per CU takes a further
-// round. The ring's k group costs more as its tiles fill the chip (its clock falls). Over those shapes the choice is
-// within 0.6% of the fastest kernel on average (at worst 15%) and never slower than the ring.
-float small_tile_us(const SmallTile& t, int64_t M, int64_t m, int64_t k) {
-  const int64_t tiles = (M + t.rows - 1) / t.rows * ((m + t.weights - 1) / t.weights);
-  const float rounds = (float)((tiles + 255) / 256), mt = t.rows / 16, n = t.weights / 16;
-  const float per_kg = -0.14f + (t.waves < 8 ? 0.2125f : 0.150f) * mt + 0.0322f * n + 0.0082f * mt * n;
-  return 2.8f + 0.75f * (rounds - 1) + rounds * (0.045f * mt * n + (float)(k / 512) * per_kg);
-}
-float ring_us(int64_t M, int64_t m, int64_t k) {
-  const int64_t tiles = (M + 127) / 128 * (m / 256);
-  const float rounds = (float)((tiles + 255) / 256), full = (float)tiles / 256.f, kg = (float)(k / 512);
-  return 1.2f + rounds * (2.7f + 1.73f * kg) + full * (3.4f + 0.71f * kg);
-}
-// the fastest small tile for M rows by the fit (null when none takes the shape), its time in *us
-const SmallTile* best_small_tile(int64_t M, int64_t m, int64_t k, float* us) {
-  const SmallTile* best = nullptr;
-  for (const SmallTile& t : kSmallTiles) {
-    if (small_tile_lds(t, k) > 163840 || (M + t.rows - 1) / t.rows > 65535) continue;
-    const float u = small_tile_us(t, M, m, k);
-    if (!best || u < *us) best = &t, *us = u;
-  }
-  return best;
-}
-// The rows the ring takes, a whole number of its 128-row blocks or all of them (the small tiles take the rest).
-// A small tile is taken where the fit has it 15% shorter (the two fits' error). Where the ring's last round is not
-// full, its whole blocks of the rounds before may stay on the ring and the rest go to small tiles: M = 1024, N = 9216,
-// K = 7168 (288 tiles, 1.1 rounds) 70.7 -> 59.3 us; M = 2048 (2.25 rounds) 117 -> 113; at 1.5 rounds and above the
-// ring alone is as fast.
-int32_t ring_rows(int64_t M, int64_t m, int64_t k) {
-  float us = 0, rest_us = 0;
-  const float ring = ring_us(M, m, k);
-  if (best_small_tile(M, m, k, &us) && us < 0.85f * ring) return 0;
-  const int64_t nb = m / 256, rounds = ((M + 127) / 128 * nb + 255) / 256;
-  const int64_t blocks = 256 * (rounds - 1) / nb;  // whole blocks in all rounds but the last
-  if (blocks > 0 && best_small_tile(M - 128 * blocks, m, k, &rest_us) &&
-      ring_us(128 * blocks, m, k) + rest_us < 0.95f * ring)
-    return (int32_t)(128 * blocks);
-  return (int32_t)M;
-}
-
+using kern::SmallTile;
 struct DenseGemm {
   const char* ring;  // the ring's entry; a small tile's is this + _t{rows}x{weights}
   const uint8_t *a, *sf_a, *b, *sf_b;
@@ -565,15 +511,15 @@ int launch_dense(const DenseGemm& G, int64_t r0, int32_t rows, const SmallTile* 
   char entry[64];
   snprintf(entry, sizeof entry, "%s_t%dx%d", G.ring, t->rows, t->weights);
   return launch(entry, (uint32_t)((G.m + t->weights - 1) / t->weights), (uint32_t)((rows + t->rows - 1) / t->rows), 1,
-                64u * (uint32_t)t->waves, stream, a, (uint32_t)small_tile_lds(*t, G.k));
+                64u * (uint32_t)t->waves, stream, a, (uint32_t)kern::small_tile_lds(*t, G.k));
 }
 int dense_gemm(const DenseGemm& G, int32_t M, void* stream) {
-  const int32_t ring = ring_rows(M, G.m, G.k);
+  const int32_t ring = (int32_t)kern::ring_rows(M, G.m, G.k);
   if (ring > 0)
     if (int rc = launch_dense(G, 0, ring, nullptr, stream)) return rc;
   if (ring == M) return KERN_OK;
-  float us = 0;
-  return launch_dense(G, ring, M - ring, best_small_tile(M - ring, G.m, G.k, &us), stream);
+  double us = 0;
+  return launch_dense(G, ring, M - ring, kern::best_small_tile(M - ring, G.m, G.k, &us), stream);
 }
 
 }  // namespace
@@ -599,6 +545,14 @@ extern "C" int kern_mxfp4_gemm_bf16(const void* a_, const void* sf_a, const void
   REQUIRE((int64_t)M * k < ((int64_t)1 << 32), "mxfp4_gemm_bf16: activations [M, k] must stay below 4 GiB (M=%d k=%d)",
           M, k);
   if (M == 0) return KERN_OK;
+  if (kern::takes_walk(M, m, k)) {
+    const int32_t hb = (int32_t)kern::walk_half_groups(m);
+    char entry[40];
+    snprintf(entry, sizeof entry, "kern_mx_gemm_bf16_s%d", k / 1024);
+    Args a;
+    a.put(a_), a.put(sf_a), a.put(b), a.put(sf_b), a.put(c), a.put(dbg), a.put(M), a.put(m), a.put(k), a.put(hb);
+    return launch(entry, (uint32_t)((m / 8 + hb - 1) / hb), 1, 1, 512, stream, a);
+  }
   return dense_gemm({"kern_mx_gemm_bf16", (const uint8_t*)a_, (const uint8_t*)sf_a, (const uint8_t*)b,
                      (const uint8_t*)sf_b, (uint8_t*)c, 2, nullptr, dbg, m, k},
                     M, stream);

@@ -596,11 +596,11 @@ const RingEntry kRingEntries[] = {
     {"kern_mx_bmm_fc2", 14, 11, 128, 10},   // b [max_slots * 128, k]
     {"kern_mx_gemm_e4m3", 10, 6, 1, 8},     // b [M, k]
     {"kern_mx_gemm_bf16", 9, 5, 1, 7},      // b [M, k]
-    {"kern_mx_gemm_bf16_s1", 9, 6, 1, 8},   // xq [M, K]
-    {"kern_mx_gemm_bf16_s2", 9, 6, 1, 8},
-    {"kern_mx_gemm_bf16_s4", 9, 6, 1, 8},
-    {"kern_mx_gemm_bf16_s7", 9, 6, 1, 8},
-    {"kern_mx_gemm_bf16_s8", 9, 6, 1, 8},
+    {"kern_mx_gemm_bf16_s1", 10, 6, 1, 8},  // xq [M, K]
+    {"kern_mx_gemm_bf16_s2", 10, 6, 1, 8},
+    {"kern_mx_gemm_bf16_s4", 10, 6, 1, 8},
+    {"kern_mx_gemm_bf16_s7", 10, 6, 1, 8},
+    {"kern_mx_gemm_bf16_s8", 10, 6, 1, 8},
     {"kern_mx_bmm_fc1", 17, -1, 0, 14},     // b [tokens, k]: bound by the buffer (the program runtime checks it)
 };
 

@@ -1,0 +1,90 @@
+// Which kernel a GEMM call launches, from its sizes alone. No HIP in here, so that the rules can be checked on the
+// CPU; kern_amd/manifest.py makes the same choices for the manifest ops.
+#pragma once
+#include <stdint.h>
+
+#include <algorithm>
+
+namespace kern {
+
+inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// The walk over the weights (kern_mx_gemm_bf16_s{k / 1024}, M <= 64, k = 1024 * {1, 2, 4, 7, 8}): about 256 workgroups
+// of 8 waves with at most nine half groups of 8 weight rows each.
+inline int64_t walk_half_groups(int64_t m) { return std::min<int64_t>(9, ceil_div(m / 8, 256)); }
+
+// Where the walk is taken, else the tiles below. Its waves split K, so it streams wide weights faster; its workgroups
+// each read all of the activations, so more rows and narrow weights favour the tiles. Both measured at 5107 shapes
+// (M = 1..64, m = 256..24576, weights from HBM and from the Infinity Cache; walk, tile in us):
+//   M = 32, m = 9216, k = 7168 12.3, 14.2; M = 16, m = 18432, k = 8192 15.8, 19.6; M = 1, m = 4096, k = 1024 3.4, 3.6;
+//   M = 16, m = 7168, k = 8192 10.1, 9.0; M = 64, m = 4096, k = 4096 9.7, 6.1; M = 64, m = 9216, k = 7168 17.3, 16.6.
+// Past m = 18432 the walk needs a second round of workgroups (M = 2, m = 22528, k = 8192: the tile takes 0.94 of it).
+// By this rule no shape is more than 2.5% slower than by the walk alone.
+inline bool takes_walk(int64_t M, int64_t m, int64_t k) {
+  if (M > 64 || k % 1024 || m > 18432) return false;
+  const int64_t ktw = k / 1024;
+  if (ktw != 1 && ktw != 2 && ktw != 4 && ktw != 7 && ktw != 8) return false;
+  const int64_t widest = M <= 16   ? (ktw == 1 ? 0 : 8192)  // the widest weights that the tiles take
+                         : M <= 32 ? (ktw == 1 ? 4096 : 8192)
+                         : ktw <= 4 ? 16384
+                         : M <= 48 ? 6144
+                                   : 8192;
+  return m > widest;
+}
+
+// The other kernels of a dense MXFP4 x MXFP8 GEMM: the small tiles (kern_mx_gemm_*_t{rows}x{weights}) and the LDS
+// ring's 128 x 256 tiles. All of these accumulate K in the same order, so the choice does not show in the results.
+struct SmallTile {
+  int rows, weights, waves, stages;
+};
+static const SmallTile kSmallTiles[] = {
+    {16, 32, 2, 8}, {16, 64, 4, 8}, {16, 128, 8, 4}, {32, 128, 8, 4}, {48, 128, 8, 4},
+    {80, 128, 8, 3}, {32, 256, 8, 3}, {48, 256, 8, 3}, {64, 256, 8, 3},
+};
+// dynamic LDS of a small tile: the activation ring, then the token scales in whole KiB
+inline int64_t small_tile_lds(const SmallTile& t, int64_t k) {
+  return (int64_t)t.stages * t.rows * 512 + ceil_div(t.rows * (k / 512 + 1), 64) * 1024;
+}
+// Microseconds of a launch, fitted to both kernels over 150 shapes (M = 17..3000, N = 512..9216, K = 512..8192,
+// graph replays; rms 10% for the tiles, 5% for the ring). A tile's k group costs by its token subtiles (mt), its
+// 16-row weight groups (n) and their product, its output by the product; a tile past one per CU takes a further
+// round. The ring's k group costs more as its tiles fill the chip (its clock falls).
+inline double small_tile_us(const SmallTile& t, int64_t M, int64_t m, int64_t k) {
+  const int64_t tiles = ceil_div(M, t.rows) * ceil_div(m, t.weights);
+  const double rounds = (double)ceil_div(tiles, 256), mt = t.rows / 16, n = t.weights / 16;
+  const double per_kg = -0.14 + (t.waves < 8 ? 0.2125 : 0.150) * mt + 0.0322 * n + 0.0082 * mt * n;
+  return 2.8 + 0.75 * (rounds - 1) + rounds * (0.045 * mt * n + (double)(k / 512) * per_kg);
+}
+inline double ring_us(int64_t M, int64_t m, int64_t k) {
+  const int64_t tiles = ceil_div(M, 128) * (m / 256);
+  const double rounds = (double)ceil_div(tiles, 256), full = (double)tiles / 256, kg = (double)(k / 512);
+  return 1.2 + rounds * (2.7 + 1.73 * kg) + full * (3.4 + 0.71 * kg);
+}
+// the fastest small tile for M rows by the fit (null when none takes the shape), its time in *us
+inline const SmallTile* best_small_tile(int64_t M, int64_t m, int64_t k, double* us) {
+  const SmallTile* best = nullptr;
+  for (const SmallTile& t : kSmallTiles) {
+    if (small_tile_lds(t, k) > 163840 || ceil_div(M, t.rows) > 65535) continue;
+    const double u = small_tile_us(t, M, m, k);
+    if (!best || u < *us) best = &t, *us = u;
+  }
+  return best;
+}
+// The rows the ring takes, a whole number of its 128-row blocks or all of them (the small tiles take the rest).
+// A small tile is taken where the fit has it 15% shorter (the two fits' error). Where the ring's last round is not
+// full, its whole blocks of the rounds before may stay on the ring and the rest go to small tiles: M = 1024, N = 9216,
+// K = 7168 (288 tiles, 1.1 rounds) 70.7 -> 59.3 us; M = 2048 (2.25 rounds) 117 -> 113; at 1.5 rounds and above the
+// ring alone is as fast.
+inline int64_t ring_rows(int64_t M, int64_t m, int64_t k) {
+  double us = 0, rest_us = 0;
+  const double ring = ring_us(M, m, k);
+  if (best_small_tile(M, m, k, &us) && us < 0.85 * ring) return 0;
+  const int64_t nb = m / 256, rounds = ceil_div(ceil_div(M, 128) * nb, 256);
+  const int64_t blocks = 256 * (rounds - 1) / nb;  // whole blocks in all rounds but the last
+  if (blocks > 0 && best_small_tile(M - 128 * blocks, m, k, &rest_us) &&
+      ring_us(128 * blocks, m, k) + rest_us < 0.95 * ring)
+    return 128 * blocks;
+  return M;
+}
+
+}  // namespace kern

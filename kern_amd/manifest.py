@@ -260,12 +260,62 @@ def mxfp4_gemv_bf16(N: int, K: int, rows_var: str = "tokens") -> dict:
             "impl": {"launches": _by_rows(lambda M: _gemv_launch(N, K, M, rows_var), rows_var, 1, GEMV_MAX_ROWS)}}
 
 
+# The small tiles of the dense GEMM: token rows, weight rows, waves, k groups of 512 in flight (csrc/pick.h)
+SMALL_TILES = ((16, 32, 2, 8), (16, 64, 4, 8), (16, 128, 8, 4), (32, 128, 8, 4), (48, 128, 8, 4), (80, 128, 8, 3),
+               (32, 256, 8, 3), (48, 256, 8, 3), (64, 256, 8, 3))
+
+
+def takes_walk(M: int, N: int, K: int) -> bool:
+    """Whether the dense bf16 GEMM runs on the walk over the weights (csrc/pick.h: takes_walk, the same rule)."""
+    if M > 64 or K % 1024 or K // 1024 not in WALK_KTW or N > 18432:
+        return False
+    if M <= 32:
+        widest = (0 if M <= 16 else 4096) if K == 1024 else 8192
+    else:
+        widest = 16384 if K <= 4096 else 6144 if M <= 48 else 8192
+    return N > widest
+
+
+def _small_tile_lds(t, K: int) -> int:
+    return t[3] * t[0] * 512 + _ceil(t[0] * (K // 512 + 1), 64) * 1024
+
+
+def _small_tile_us(t, M: int, N: int, K: int) -> float:
+    rows, weights, waves, _ = t
+    rounds, mt, n = _ceil(_ceil(M, rows) * _ceil(N, weights), 256), rows // 16, weights // 16
+    per_kg = -0.14 + (0.2125 if waves < 8 else 0.150) * mt + 0.0322 * n + 0.0082 * mt * n
+    return 2.8 + 0.75 * (rounds - 1) + rounds * (0.045 * mt * n + K // 512 * per_kg)
+
+
+def best_small_tile(M: int, N: int, K: int):
+    """The small tile that the fit of csrc/pick.h has as the fastest."""
+    return min((t for t in SMALL_TILES if _small_tile_lds(t, K) <= 163840), key=lambda t: _small_tile_us(t, M, N, K))
+
+
+def _small_gemm_launch(N: int, K: int, M: int, rows_var: str) -> dict:
+    """The launch kern_mxfp4_gemm_bf16 makes for M <= 64 rows (csrc/capi.cpp) at the walk's K."""
+    p = ["in buffer<u8>"] * 4 + ["out buffer<bf16>"]
+    a = [{"param": i} for i in range(5)]
+    if takes_walk(M, N, K):
+        H = N // 8
+        hb = min(9, _ceil(H, 256))
+        return {"entry": f"kern_mx_gemm_bf16_s{K // 1024}", "params": p + ["i64", "bytes<4>", "i32", "i32", "i32"],
+                "block": [512, 1, 1], "grid": [_ceil(H, hb), 1, 1],
+                "args": a + [{"i64": 0}, _rows(rows_var), {"i32": N}, {"i32": K}, {"i32": hb}]}
+    t = best_small_tile(M, N, K)
+    rows, weights, waves, _ = t
+    return {"entry": f"kern_mx_gemm_bf16_t{rows}x{weights}", "params": p + ["bytes<4>", "i32", "i32", "i64"],
+            "block": [64 * waves, 1, 1], "grid": [_ceil(N, weights), {"ceil_div": [rows_var, rows]}, 1],
+            "shared_mem": _small_tile_lds(t, K), "args": a + [_rows(rows_var), {"i32": N}, {"i32": K}, {"i64": 0}]}
+
+
 def mxfp4_gemm_bf16(N: int, K: int, rows_var: str = "tokens") -> dict:
     """The dense MXFP4 x MXFP8 GEMM with bf16 out (C ABI kern_mxfp4_gemm_bf16): in u8 a [N][K/2], sf_a (the
     repacked weights), b [M][K] and sf_b (MXFP8 activations, linear scales), out bf16 c [M][N]; M = the value
-    of `rows_var`. Up to 64 rows the 32 x 128 tiles (K = 1024 * {1, 2, 4, 7, 8}), else the ring's 128 x 256 ones,
-    grid [N/256, ceil(M/128)]; both with a null f32 debug pointer. The C ABI chooses among more tile shapes; every
-    kernel of the family accumulates K in the same order, so the bits are the same."""
+    of `rows_var`. Up to 64 rows, at K = 1024 * {1, 2, 4, 7, 8}, the walk over the weights or a small tile, as the C
+    ABI chooses by M (one launch per run of M that takes the same kernel), else the ring's 128 x 256 tiles, grid
+    [N/256, ceil(M/128)]; all with a null f32 debug pointer. Where the C ABI takes small tiles for other K or more
+    rows the ring's bits are the same."""
     assert N % 256 == 0 and K % 512 == 0
     p = ["in buffer<u8>"] * 4 + ["out buffer<bf16>"]
     tiled = {"module": MODULE, "entry": "kern_mx_gemm_bf16", "params": p + ["bytes<4>", "i32", "i32", "i64"],
@@ -273,12 +323,8 @@ def mxfp4_gemm_bf16(N: int, K: int, rows_var: str = "tokens") -> dict:
              "args": [{"param": i} for i in range(5)] + [_rows(rows_var), {"i32": N}, {"i32": K}, {"i64": 0}]}
     if not (K % 1024 == 0 and K // 1024 in WALK_KTW):
         return {"params": p, "impl": {"launches": [tiled]}}
-    small = {"module": MODULE, "entry": f"kern_mx_gemm_bf16_s{K // 1024}",
-             "params": p + ["i64", "bytes<4>", "i32", "i32"], "block": [512, 1, 1],
-             "grid": [N // 128, {"ceil_div": [rows_var, 32]}, 1], "when": {"var": rows_var, "max": 64},
-             "shared_mem": 4 * 16384 + _ceil(32 * (K // 512 + 1), 64) * 1024,  # kSmallTiles' {32, 128} (capi.cpp)
-             "args": [{"param": i} for i in range(5)] + [{"i64": 0}, _rows(rows_var), {"i32": N}, {"i32": K}]}
-    return {"params": p, "impl": {"launches": [small, {**tiled, "when": {"var": rows_var, "min": 65}}]}}
+    small = _by_rows(lambda M: _small_gemm_launch(N, K, M, rows_var), rows_var, 1, 64)
+    return {"params": p, "impl": {"launches": small + [{**tiled, "when": {"var": rows_var, "min": 65}}]}}
 
 
 def mxfp4_gemm_e4m3(N: int, K: int, rows_var: str = "tokens") -> dict:

@@ -107,3 +107,38 @@ def test_mxfp8_tiles(ops, oracle, rows, weights):
         assert (got[:, N:] == 7.0).all() and (got[M] == 7.0).all()
         assert_gemm_close(got[:M, :N], oracle.mxfp8_gemm(qa, qw, ta, tw, M, N, K), f"{rows}x{weights} {M}x{N}x{K}")
     mod.close()
+
+
+@pytest.mark.parametrize("N,K,hb", [(256, 1024, 1), (4352, 2048, 3), (2304, 4096, 9), (9216, 7168, 5), (512, 8192, 2)])
+def test_saved_walk_launch(ops, oracle, N, K, hb):
+    """The walk (kern_mx_gemm_bf16_s{K / 1024}) as a manifest op saved before there were tiles launches it, with any share
+    of half groups: against the oracle at ragged token counts."""
+    from tests.test_pick import saved_walk_op
+
+    op = ops.ManifestOp(saved_walk_op(N, K, hb))
+    for M in (1, 17, 50, 64):
+        print(f"[walk] M={M} N={N} K={K} hb={hb}", flush=True)
+        w, s, q, qs = _operands(ops, M, N, K, 90)
+        c = torch.full((M + 1, N), 7.0, dtype=torch.bfloat16, device="cuda")
+        op(w, s, q, qs, c, vars={"tokens": M})
+        torch.cuda.synchronize()
+        got = bf16_to_f32(to_np(c))
+        assert (got[M] == 7.0).all()
+        _, acc = oracle.gemm_e4m3_pt(to_np(w), to_np(s), to_np(q), to_np(qs), N, K, 1.0)
+        assert_gemm_close(got[:M], acc, f"walk {M}x{N}x{K}")
+
+
+@pytest.mark.parametrize("N,K", [(2048, 8192), (4352, 1024), (7168, 8192), (8448, 4096), (18688, 1024)])
+def test_dense_op_has_the_c_abi_bits_up_to_64_rows(ops, N, K):
+    """Each launch of the manifest op at the edges of its rows: the walk where the C ABI takes it, else the ring's bits."""
+    from kern_amd import manifest as mf
+
+    op = ops.ManifestOp(mf.mxfp4_gemm_bf16(N, K))
+    w, s, q, qs = _operands(ops, 65, N, K, 95)
+    for M in (1, 16, 17, 32, 33, 48, 49, 64, 65):
+        print(f"[dense op] M={M} N={N} K={K}", flush=True)
+        c, m = (torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+        ops.mxfp4_gemm_bf16(w, s, q[:M], qs[:M], c, M=M, m=N, k=K)
+        op(w, s, q[:M], qs[:M], m, vars={"tokens": M})
+        torch.cuda.synchronize()
+        assert torch.equal(c.view(torch.int16), m.view(torch.int16)), M

@@ -1,0 +1,113 @@
+"""The rules that choose a GEMM's kernel (kern_amd/csrc/pick.h), compiled on the host: the manifest ops' copy of them
+agrees, and at shapes with measured times the choice is no slower than the kernel that the same call ran on before
+there was one to make."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+from kern_amd import build as kb
+from kern_amd import manifest as mf
+from kern_amd import ops
+
+SHIM = """
+#include "pick.h"
+using namespace kern;
+extern "C" int takes(int64_t M, int64_t m, int64_t k) { return takes_walk(M, m, k); }
+extern "C" int tile(int64_t M, int64_t m, int64_t k, int* rows, int* weights, int64_t* lds) {
+  double us = 0;
+  const SmallTile* t = best_small_tile(M, m, k, &us);
+  if (!t) return 0;
+  *rows = t->rows, *weights = t->weights, *lds = small_tile_lds(*t, k);
+  return 1;
+}
+extern "C" int64_t ring(int64_t M, int64_t m, int64_t k) { return ring_rows(M, m, k); }
+"""
+
+
+@pytest.fixture(scope="module")
+def pick(tmp_path_factory):
+    d = tmp_path_factory.mktemp("pick")
+    (d / "shim.cpp").write_text(SHIM)
+    csrc = os.path.join(os.path.dirname(kb.__file__), "csrc")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", f"-I{csrc}", str(d / "shim.cpp"), "-o",
+                    str(d / "shim.so")], check=True)
+    L = ctypes.CDLL(str(d / "shim.so"))
+    L.ring.restype = ctypes.c_int64
+    for f in (L.takes, L.ring):
+        f.argtypes = [ctypes.c_int64] * 3
+    L.tile.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_void_p] * 3
+    return L
+
+
+def tile_of(pick, M, N, K):
+    r, w, lds = ctypes.c_int(), ctypes.c_int(), ctypes.c_int64()
+    return (r.value, w.value, lds.value) if pick.tile(M, N, K, ctypes.byref(r), ctypes.byref(w), ctypes.byref(lds)) \
+        else None
+
+
+def dense_route(pick, M, N, K, out="bf16"):
+    """What a dense call launches: "walk", "ring", a tile "t{rows}x{weights}", or "split"."""
+    if out == "bf16" and pick.takes(M, N, K):
+        return "walk"
+    ring = pick.ring(M, N, K)
+    return "ring" if ring == M else "split" if ring else "t%dx%d" % tile_of(pick, M, N, K)[:2]
+
+
+def test_manifest_makes_the_same_dense_choice(pick):
+    for K in (1024, 2048, 4096, 7168, 8192):
+        for N in [256 * i for i in range(1, 40)] + [14336, 16384, 16640, 18432, 18688, 24576]:
+            for M in (1, 2, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64):
+                want = f"kern_mx_gemm_bf16_s{K // 1024}" if pick.takes(M, N, K) else \
+                    "kern_mx_gemm_bf16_t%dx%d" % tile_of(pick, M, N, K)[:2]
+                L = mf._small_gemm_launch(N, K, M, "tokens")
+                assert L["entry"] == want, (M, N, K)
+                if "_t" in want:
+                    assert L["shared_mem"] == tile_of(pick, M, N, K)[2] <= 163840
+
+
+# M, N, K, microseconds of the walk and of the tile that the fit picks (weights from HBM or from the Infinity Cache)
+WALK_TIMES = [
+    (16, 9216, 7168, 9.98, 11.11), (17, 9216, 8192, 12.59, 14.79), (32, 9216, 7168, 12.33, 14.21),
+    (16, 18432, 8192, 15.82, 19.64), (37, 17920, 7168, 17.99, 24.61), (64, 18432, 7168, 21.82, 27.17),
+    (40, 18432, 4096, 13.42, 14.36), (16, 9216, 1024, 4.09, 4.48), (1, 4096, 1024, 3.38, 3.61),
+    (64, 18432, 2048, 10.52, 11.53), (16, 7168, 8192, 10.12, 8.97), (64, 4096, 4096, 9.73, 6.09),
+    (64, 2048, 8192, 14.68, 6.35), (32, 1024, 4096, 6.71, 4.42), (48, 9216, 2048, 7.22, 5.26),
+    (64, 256, 1024, 5.61, 3.30), (2, 22528, 8192, 23.17, 21.79),
+]
+
+
+@pytest.mark.parametrize("M,N,K,walk,tile", WALK_TIMES)
+def test_walk_where_it_is_faster(pick, M, N, K, walk, tile):
+    """Up to 64 rows the walk is what every such call ran on before the tiles: the choice is within 3% of it."""
+    route = dense_route(pick, M, N, K)
+    assert (walk if route == "walk" else tile) <= 1.03 * walk, route
+
+
+@pytest.mark.parametrize("K", [1024, 2048, 4096, 7168, 8192])
+def test_walk_launch_of_a_saved_op_is_accepted(K):
+    """A manifest op that launches the walk with its arguments as they always were (dbg, M, m, k, hb; one-dimensional
+    grid, static LDS) matches the code object's metadata, and plans."""
+    if not os.path.exists(ops.LIB_PATH):
+        pytest.skip("library not built (python -m kern_amd.build)")
+    N, entry = 9216, f"kern_mx_gemm_bf16_s{K // 1024}"
+    params = ["in buffer<u8>"] * 4 + ["out buffer<bf16>", "i64", "bytes<4>", "i32", "i32", "i32"]
+    with open(ops.HSACO_PATH, "rb") as f:
+        img = f.read()
+    sizes, n = (ctypes.c_uint32 * 32)(), ctypes.c_int()
+    assert ops.lib().kern_code_object_param_sizes(img, len(img), entry.encode(), sizes, 32, ctypes.byref(n)) == 0
+    assert list(sizes[:n.value]) == [8] * 6 + [4] * 4
+    op = saved_walk_op(N, K, 5)
+    p = ops.op_plan(op, 0, [0x1000 * (i + 1) for i in range(5)], {"tokens": 33})
+    assert not p["skip"] and p["grid"] == (-(-N // 8 // 5), 1, 1) and p["shared"] == 0
+
+
+def saved_walk_op(N, K, hb):
+    p = ["in buffer<u8>"] * 4 + ["out buffer<bf16>"]
+    return {"params": p, "impl": {"launches": [{
+        "module": mf.MODULE, "entry": f"kern_mx_gemm_bf16_s{K // 1024}",
+        "params": p + ["i64", "bytes<4>", "i32", "i32", "i32"], "block": [512, 1, 1], "grid": [-(-N // 8 // hb), 1, 1],
+        "when": {"var": "tokens", "max": 64},
+        "args": [{"param": i} for i in range(5)] + [{"i64": 0}, mf._rows("tokens"), {"i32": N}, {"i32": K},
+                                                    {"i32": hb}]}]}}
