@@ -45,19 +45,30 @@ static const SmallTile kSmallTiles[] = {
 inline int64_t small_tile_lds(const SmallTile& t, int64_t k) {
   return (int64_t)t.stages * t.rows * 512 + ceil_div(t.rows * (k / 512 + 1), 64) * 1024;
 }
-// Microseconds of a launch, fitted to both kernels over 150 shapes (M = 17..3000, N = 512..9216, K = 512..8192,
-// graph replays; rms 10% for the tiles, 5% for the ring). A tile's k group costs by its token subtiles (mt), its
-// 16-row weight groups (n) and their product, its output by the product; a tile past one per CU takes a further
-// round. The ring's k group costs more as its tiles fill the chip (its clock falls).
+// Microseconds of a launch, fitted to both kernels over 150 shapes (M = 17..3000, N = 512..9216, K = 512..8192, graph
+// replays) and corrected where 6184 more (M = 1..6144, N = 256..20480, K = 512..16384, weights from HBM and from the
+// Infinity Cache) showed a bias. A tile's k group costs by its token subtiles (mt), its 16-row weight groups (n) and
+// their product, its output by the product; a tile past one per CU takes a further round. Tiles that fill the chip
+// are slower by a tenth, and by 40% more where K/512 is 7, 15 or 31: the weight rows of its waves then lie a power of
+// two less 4 KiB apart, and their requests meet on the same channels (32 x 128 to 80 x 128 tiles on 180 to 256 CUs:
+// 1.3, 1.6 and 1.65 times the fit, against 1.1 to 1.2 at other K).
 inline double small_tile_us(const SmallTile& t, int64_t M, int64_t m, int64_t k) {
-  const int64_t tiles = ceil_div(M, t.rows) * ceil_div(m, t.weights);
+  const int64_t tiles = ceil_div(M, t.rows) * ceil_div(m, t.weights), kg = k / 512;
   const double rounds = (double)ceil_div(tiles, 256), mt = t.rows / 16, n = t.weights / 16;
   const double per_kg = -0.14 + (t.waves < 8 ? 0.2125 : 0.150) * mt + 0.0322 * n + 0.0082 * mt * n;
-  return 2.8 + 0.75 * (rounds - 1) + rounds * (0.045 * mt * n + (double)(k / 512) * per_kg);
+  const double us = 2.8 + 0.75 * (rounds - 1) + rounds * (0.045 * mt * n + (double)kg * per_kg);
+  const double full = std::min(1.0, (double)tiles / 256);
+  return us * (1 + 0.1 * full) * (kg >= 7 && (kg & (kg + 1)) == 0 ? 1 + 0.4 * full : 1);
 }
+// The ring's k group costs more as its tiles fill the chip (its clock falls). A last round that holds only tiles of a
+// partial block of rows costs their share of the rows, 0.3 at least (M = 531, N = 13312, K = 10240, 52 tiles of 19 rows
+// after 208 whole ones: 65 us against the 94 of two whole rounds).
 inline double ring_us(int64_t M, int64_t m, int64_t k) {
-  const int64_t tiles = ceil_div(M, 128) * (m / 256);
-  const double rounds = (double)ceil_div(tiles, 256), full = (double)tiles / 256, kg = (double)(k / 512);
+  const int64_t nb = m / 256, tiles = ceil_div(M, 128) * nb, part = M % 128;
+  double rounds = (double)ceil_div(tiles, 256);
+  if (part && rounds > 1 && M / 128 * nb <= 256 * ((int64_t)rounds - 1))
+    rounds += std::max(0.3, (double)part / 128) - 1;
+  const double full = (double)tiles / 256, kg = (double)(k / 512);
   return 1.2 + rounds * (2.7 + 1.73 * kg) + full * (3.4 + 0.71 * kg);
 }
 // the fastest small tile for M rows by the fit (null when none takes the shape), its time in *us
@@ -71,18 +82,21 @@ inline const SmallTile* best_small_tile(int64_t M, int64_t m, int64_t k, double*
   return best;
 }
 // The rows the ring takes, a whole number of its 128-row blocks or all of them (the small tiles take the rest).
-// A small tile is taken where the fit has it 15% shorter (the two fits' error). Where the ring's last round is not
-// full, its whole blocks of the rounds before may stay on the ring and the rest go to small tiles: M = 1024, N = 9216,
-// K = 7168 (288 tiles, 1.1 rounds) 70.7 -> 59.3 us; M = 2048 (2.25 rounds) 117 -> 113; at 1.5 rounds and above the
-// ring alone is as fast.
+// A small tile is taken where the fit has it 10% shorter. Over the 6184 shapes the choice is within 0.5% of the fastest
+// kernel on average, and 3.3% slower than the ring at worst. Where the ring's last round is not full, its whole blocks
+// of the rounds before may stay on the ring and the rest go to small tiles, in a launch of their own behind the
+// ring's: taken where the fit has the two 13% shorter, which over 357 shapes with more than one round was 34 times,
+// 3% to 27% shorter measured and 13% on average (M = 1024, N = 9216, K = 7168, 288 tiles: 70.7 -> 59.3 us). With 5%
+// asked for it was 124 times, up to 14% slower (M = 531, N = 13312, K = 10240), and level at M = 2048, N = 9216,
+// K = 7168 (2.25 rounds).
 inline int64_t ring_rows(int64_t M, int64_t m, int64_t k) {
   double us = 0, rest_us = 0;
   const double ring = ring_us(M, m, k);
-  if (best_small_tile(M, m, k, &us) && us < 0.85 * ring) return 0;
+  if (best_small_tile(M, m, k, &us) && us < 0.9 * ring) return 0;
   const int64_t nb = m / 256, rounds = ceil_div(ceil_div(M, 128) * nb, 256);
   const int64_t blocks = 256 * (rounds - 1) / nb;  // whole blocks in all rounds but the last
   if (blocks > 0 && best_small_tile(M - 128 * blocks, m, k, &rest_us) &&
-      ring_us(128 * blocks, m, k) + rest_us < 0.95 * ring)
+      ring_us(128 * blocks, m, k) + rest_us < 0.87 * ring)
     return 128 * blocks;
   return M;
 }

@@ -282,9 +282,11 @@ def _small_tile_lds(t, K: int) -> int:
 
 def _small_tile_us(t, M: int, N: int, K: int) -> float:
     rows, weights, waves, _ = t
-    rounds, mt, n = _ceil(_ceil(M, rows) * _ceil(N, weights), 256), rows // 16, weights // 16
+    tiles, kg, mt, n = _ceil(M, rows) * _ceil(N, weights), K // 512, rows // 16, weights // 16
+    rounds, full = _ceil(tiles, 256), min(1.0, tiles / 256)
     per_kg = -0.14 + (0.2125 if waves < 8 else 0.150) * mt + 0.0322 * n + 0.0082 * mt * n
-    return 2.8 + 0.75 * (rounds - 1) + rounds * (0.045 * mt * n + K // 512 * per_kg)
+    us = 2.8 + 0.75 * (rounds - 1) + rounds * (0.045 * mt * n + kg * per_kg)
+    return us * (1 + 0.1 * full) * (1 + 0.4 * full if kg >= 7 and kg & (kg + 1) == 0 else 1)
 
 
 def best_small_tile(M: int, N: int, K: int):

@@ -142,3 +142,25 @@ def test_dense_op_has_the_c_abi_bits_up_to_64_rows(ops, N, K):
         op(w, s, q[:M], qs[:M], m, vars={"tokens": M})
         torch.cuda.synchronize()
         assert torch.equal(c.view(torch.int16), m.view(torch.int16)), M
+
+
+@pytest.mark.parametrize("M,N,K", [(2446, 3584, 1024), (1410, 6144, 1536)])  # "split" in test_pick.py's test_dense_routes
+@pytest.mark.parametrize("dbg", [False, True])
+def test_split_has_the_rings_bits(ops, oracle, M, N, K, dbg):
+    """Whole rounds on the ring and the remaining rows on small tiles, in both outputs, against the ring alone: every
+    operand's and output's offset of the second launch."""
+    print(f"[split] M={M} N={N} K={K}", flush=True)
+    mod = ops.Module(ops.HSACO_PATH)
+    w, s, q, qs = _operands(ops, M, N, K, 70)
+    ds = torch.tensor([1.0 / 16], dtype=torch.float32, device="cuda")
+    for out, fn, extra in ((torch.bfloat16, ops.mxfp4_gemm_bf16, ()), (torch.uint8, ops.mxfp4_gemm_e4m3, (ds,))):
+        ring, got = (torch.full((M + 1, N), 77, dtype=out, device="cuda") for _ in range(2))
+        acc = [torch.full((M + 1, N), 7.0, dtype=torch.float32, device="cuda") for _ in range(2)] if dbg else [0, None]
+        name = "kern_mx_gemm_" + ("bf16" if out == torch.bfloat16 else "e4m3")
+        mod.launch(name, (N // 256, -(-M // 128)), (512,), w, s, q, qs, ring, *extra, M, N, K, acc[0])
+        fn(w, s, q, qs, got, *extra, M=M, m=N, k=K, dbg=acc[1])
+        torch.cuda.synchronize()
+        assert torch.equal(ring.view(torch.uint8), got.view(torch.uint8)), name
+        if dbg:
+            assert torch.equal(acc[0], acc[1]), name
+    mod.close()

@@ -3,6 +3,7 @@ agrees, and at shapes with measured times the choice is no slower than the kerne
 there was one to make."""
 import ctypes
 import os
+import random
 import subprocess
 
 import pytest
@@ -83,6 +84,52 @@ def test_walk_where_it_is_faster(pick, M, N, K, walk, tile):
     """Up to 64 rows the walk is what every such call ran on before the tiles: the choice is within 3% of it."""
     route = dense_route(pick, M, N, K)
     assert (walk if route == "walk" else tile) <= 1.03 * walk, route
+
+
+# M, N, K, microseconds of the ring alone and of the small tile or (split) ring and small tile that was taken before
+RING_TIMES = [
+    (388, 17664, 2048, 21.17, 29.34), (531, 13312, 10240, 64.84, 89.38), (5391, 1536, 2048, 22.42, 29.64),
+    (422, 17152, 1024, 16.47, 18.77), (2237, 1024, 15872, 62.69, 71.31), (1973, 2048, 3584, 19.16, 21.65),
+    (567, 5632, 7680, 34.74, 40.84), (3360, 768, 7680, 32.02, 36.81), (2394, 1024, 7680, 31.98, 36.64),
+    (3235, 2560, 1536, 19.59, 21.91), (1025, 7680, 7680, 57.18, 79.54), (555, 6400, 15872, 63.8, 78.72),
+    (550, 13568, 3584, 32.91, 41.54), (779, 9728, 4608, 37.74, 45.26), (305, 11776, 7680, 38.26, 45.48),
+    (1191, 7680, 512, 13.28, 15.46), (3885, 3072, 3072, 34.84, 37.59), (1813, 13312, 4608, 83.44, 96.02),
+]
+
+
+@pytest.mark.parametrize("out", ["bf16", "e4m3"])
+@pytest.mark.parametrize("M,N,K,ring,other", RING_TIMES)
+def test_ring_where_it_is_faster(pick, M, N, K, ring, other, out):
+    """The ring is what every such call ran on before the tiles (these came out slower: a chip full of large tiles, K of
+    a power of two less 512, a ring's last round of a few rows). Another tile or split may still be taken, unless it is
+    what was measured."""
+    route = dense_route(pick, M, N, K, out)
+    assert other > 1.03 * ring and route == "ring", route
+
+
+# M, N, K whose gain is to stay: a tile against the ring (M > 64, or K without the walk), and ring rounds with tiles after
+@pytest.mark.parametrize("M,N,K,route", [(40, 6144, 3584, "tile"), (200, 4096, 7168, "tile"), (200, 7168, 2048, "tile"),
+                                         (128, 9216, 7168, "tile"), (17, 512, 512, "tile"), (1024, 9216, 7168, "split"),
+                                         (2446, 3584, 1024, "split"), (1410, 6144, 1536, "split"),
+                                         (2048, 9216, 7168, "ring"),
+                                         (4096, 2048, 7168, "ring"), (2048, 7168, 8192, "ring")])
+def test_dense_routes(pick, M, N, K, route):
+    got = dense_route(pick, M, N, K, "e4m3")
+    assert got == route or (route == "tile" and got[0] == "t"), got
+
+
+def test_split_is_whole_blocks_and_leaves_rows(pick):
+    """Over the declared range: the ring's rows are none, all, or whole blocks short of all."""
+    rng = random.Random(3)
+    seen = set()
+    for _ in range(20000):
+        M, N, K = rng.randint(1, 6000), 256 * rng.randint(1, 80), 512 * rng.randint(1, 32)
+        r = pick.ring(M, N, K)
+        assert r == M or (r % 128 == 0 and 0 <= r < M)
+        seen.add("ring" if r == M else "split" if r else "tile")
+        if r < M:
+            assert tile_of(pick, M - r, N, K)[2] <= 163840
+    assert seen == {"ring", "split", "tile"}
 
 
 @pytest.mark.parametrize("K", [1024, 2048, 4096, 7168, 8192])
