@@ -666,35 +666,6 @@ extern "C" int kern_moe_finalize(const void* fc2_out, const int32_t* exp2perm, c
   return launch("kern_mx_moe_finalize", (uint32_t)tokens, 1, 1, 256, stream, a);
 }
 
-namespace {
-
-// Small tiles of the MXFP8 x MXFP8 GEMM (kern_mx_gemm_mxfp8_t{rows}x{weights}); the fit of their times and of
-// kern_mx_gemm_mxfp8's is over 78 shapes (M = 16..1187, N = 512..9216, K = 512..7936; rms 11% and 8%). A tile costs by
-// its token subtiles (mt) and 16-row weight groups (n) for every eight k-tiles, one of each wave. A tile is taken where
-// the fit has it 15% shorter (its error): over those shapes 1% slower than the fastest kernel on average, 26% at worst,
-// and never slower than the large tiles.
-struct SmallTile8 {
-  int rows, weights;
-};
-const SmallTile8 kSmallTiles8[] = {{16, 16}, {16, 32}, {16, 64}, {32, 64}, {32, 128}, {48, 64}, {64, 64}};
-const SmallTile8* small_tile8(int64_t m, int64_t n, int64_t k) {
-  const int64_t kt = (k + 127) / 128, big = (m + 127) / 128 * ((n + 255) / 256);
-  const float large = 5.2f + 0.93f * (float)((big + 255) / 256) * kt + (float)big / 256.f * (8.4f + 0.134f * kt);
-  const SmallTile8* best = nullptr;
-  float us = 0.85f * large;
-  for (const SmallTile8& t : kSmallTiles8) {
-    const int64_t tiles = (m + t.rows - 1) / t.rows * ((n + t.weights - 1) / t.weights);
-    if ((m + t.rows - 1) / t.rows > 65535 || k > 1 << 20) continue;  // grid.y; 32-bit offsets within a tile
-    const float rounds = (float)((tiles + 255) / 256), mt = t.rows / 16, ng = t.weights / 16;
-    const float per8 = -0.046f + 0.304f * mt + 0.176f * ng + 0.0054f * mt * ng;
-    const float u = 1.8f + 0.11f * (rounds - 1) + rounds * (0.075f * mt * ng + (float)((kt + 7) / 8) * per8);
-    if (u < us) best = &t, us = u;
-  }
-  return best;
-}
-
-}  // namespace
-
 extern "C" int kern_mxfp8_gemm_bf16(const void* a, const void* w, void* c, const void* a_sf, const void* w_sf, int32_t m,
                                     int32_t n, int32_t k, int32_t ldc, void* stream) {
   REQUIRE(m >= 0 && n >= 0 && k >= 0 && k % 32 == 0 && ldc >= n,
@@ -706,7 +677,7 @@ extern "C" int kern_mxfp8_gemm_bf16(const void* a, const void* w, void* c, const
   if (k == 0) return fail(KERN_ERR_API, "cublaslt_mxfp8_tn: k == 0 leaves c undefined; zero it instead");
   Args x;
   x.put(a), x.put(w), x.put(c), x.put(a_sf), x.put(w_sf), x.put(m), x.put(n), x.put(k), x.put(ldc);
-  if (const SmallTile8* t = small_tile8(m, n, k)) {
+  if (const kern::SmallTile8* t = kern::small_tile8(m, n, k)) {
     char entry[64];
     snprintf(entry, sizeof entry, "kern_mx_gemm_mxfp8_t%dx%d", t->rows, t->weights);
     const uint32_t mt = (uint32_t)t->rows / 16, ng = (uint32_t)t->weights / 16;

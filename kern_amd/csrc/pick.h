@@ -101,4 +101,32 @@ inline int64_t ring_rows(int64_t M, int64_t m, int64_t k) {
   return M;
 }
 
+// Small tiles of the MXFP8 x MXFP8 GEMM (kern_mx_gemm_mxfp8_t{rows}x{weights}); the fit of their times and of
+// kern_mx_gemm_mxfp8's is over 78 shapes (M = 16..1187, N = 512..9216, K = 512..7936; rms 11% and 8%). A tile costs by
+// its token subtiles (mt) and 16-row weight groups (n) for every eight k-tiles, one of each wave. A tile is taken where
+// the fit has it 15% shorter (its error), in three and more rounds 28% (there its error grows: M = 524, N = 7296,
+// K = 960, 1254 tiles of 48 x 64 took 23.0 us against the large tiles' 18.6). Over 8582 shapes (M = 1..6144,
+// N = 16..20480, K = 128..16384) the choice takes 0.34 of the large tiles' time, is within 1% of the fastest on average,
+// and never slower than the large tiles; with 15% at any number of rounds 16 were, by up to 24%.
+struct SmallTile8 {
+  int rows, weights;
+};
+static const SmallTile8 kSmallTiles8[] = {{16, 16}, {16, 32}, {16, 64}, {32, 64}, {32, 128}, {48, 64}, {64, 64}};
+inline const SmallTile8* small_tile8(int64_t m, int64_t n, int64_t k) {
+  const int64_t kt = ceil_div(k, 128), big = ceil_div(m, 128) * ceil_div(n, 256);
+  const double large =
+      5.2 + 0.93 * (double)ceil_div(big, 256) * (double)kt + (double)big / 256 * (8.4 + 0.134 * (double)kt);
+  const SmallTile8* best = nullptr;
+  double us = 0, most = 0;  // the fastest tile's time, and the longest with which a tile of its rounds is taken
+  for (const SmallTile8& t : kSmallTiles8) {
+    if (ceil_div(m, t.rows) > 65535 || k > 1 << 20) continue;  // grid.y; 32-bit offsets within a tile
+    const double rounds = (double)ceil_div(ceil_div(m, t.rows) * ceil_div(n, t.weights), 256);
+    const double mt = t.rows / 16, ng = t.weights / 16;
+    const double per8 = -0.046 + 0.304 * mt + 0.176 * ng + 0.0054 * mt * ng;
+    const double u = 1.8 + 0.11 * (rounds - 1) + rounds * (0.075 * mt * ng + (double)ceil_div(kt, 8) * per8);
+    if (!best || u < us) best = &t, us = u, most = (rounds <= 2 ? 0.85 : 0.72) * large;
+  }
+  return best && us < most ? best : nullptr;
+}
+
 }  // namespace kern

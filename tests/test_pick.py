@@ -23,6 +23,10 @@ extern "C" int tile(int64_t M, int64_t m, int64_t k, int* rows, int* weights, in
   *rows = t->rows, *weights = t->weights, *lds = small_tile_lds(*t, k);
   return 1;
 }
+extern "C" int tile8(int64_t m, int64_t n, int64_t k) {
+  const SmallTile8* t = small_tile8(m, n, k);
+  return t ? t->rows * 1000 + t->weights : 0;
+}
 extern "C" int64_t ring(int64_t M, int64_t m, int64_t k) { return ring_rows(M, m, k); }
 """
 
@@ -36,7 +40,7 @@ def pick(tmp_path_factory):
                     str(d / "shim.so")], check=True)
     L = ctypes.CDLL(str(d / "shim.so"))
     L.ring.restype = ctypes.c_int64
-    for f in (L.takes, L.ring):
+    for f in (L.takes, L.ring, L.tile8):
         f.argtypes = [ctypes.c_int64] * 3
     L.tile.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_void_p] * 3
     return L
@@ -130,6 +134,22 @@ def test_split_is_whole_blocks_and_leaves_rows(pick):
         if r < M:
             assert tile_of(pick, M - r, N, K)[2] <= 163840
     assert seen == {"ring", "split", "tile"}
+
+
+@pytest.mark.parametrize("M,N,K,large,tile", [
+    (524, 7296, 960, 18.59, 23.03), (644, 5384, 960, 17.61, 19.67), (2367, 1664, 992, 18.72, 20.65),
+    (2932, 976, 3840, 37.27, 40.48), (144, 18464, 2688, 30.14, 32.59), (399, 7320, 704, 14.59, 15.72),
+    (3070, 792, 4992, 40.54, 44.91), (4050, 688, 4992, 40.99, 46.99)])
+def test_mxfp8_large_tiles_where_they_are_faster(pick, M, N, K, large, tile):
+    """kern_mx_gemm_mxfp8 is what every such call ran on before the small tiles (microseconds of both)."""
+    assert tile > 1.03 * large and not pick.tile8(M, N, K)
+
+
+@pytest.mark.parametrize("M,N,K,small", [(72, 9216, 7168, True), (16, 4096, 2048, True), (200, 4096, 7168, True),
+                                         (500, 4096, 2048, True), (1, 16, 32, True), (1500, 4096, 7168, False),
+                                         (2048, 2048, 7168, False), (4096, 2048, 7168, False), (300, 520, 2 << 20, False)])
+def test_mxfp8_routes(pick, M, N, K, small):
+    assert bool(pick.tile8(M, N, K)) == small
 
 
 @pytest.mark.parametrize("K", [1024, 2048, 4096, 7168, 8192])
