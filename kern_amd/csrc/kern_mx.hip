@@ -380,8 +380,9 @@ extern "C" __global__ __launch_bounds__(256) void kern_mx_gemv_bf16_rg(
 // ranges, not whole 512-wide groups) and its loop is unrolled, so the weight stream has no requests past
 // its end and no branches around them: every request is one the compiler's wait counts can see, and an
 // extra request per wave costs measurably (one unneeded 256 B scale fragment per wave: +0.8 us at N =
-// 18432). The wave's scale fragments (those its k-tiles touch, at most five) go into LDS with one
-// buffer->LDS request beside its x slice; each k-tile reads its scale byte from there.
+// 18432). The wave's scale fragments (those its k-tiles touch, at most four, five at NKT = 15) go into LDS
+// with one buffer->LDS request (two at NKT = 15) beside its x slice; each k-tile reads its scale byte from
+// there.
 template <int NKT>
 KERN_DEV void gemv_rows_fixed(const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
                               const uint8_t* __restrict__ wsf, uint16_t* __restrict__ y, int M, int N, int K) {
@@ -405,7 +406,9 @@ KERN_DEV void gemv_rows_fixed(const uint16_t* __restrict__ x, const uint8_t* __r
   const __amdgpu_buffer_rsrc_t sr =
       __builtin_amdgcn_make_buffer_rsrc((void*)(wsf + (int64_t)rg * KG * 256), (short)0, KG * 256, 0x00020000);
   if (lane < ns * 16) __builtin_amdgcn_raw_ptr_buffer_load_lds(sr, (lds_void_t*)&ssc[wave][0], 16, kgA * 256 + lane * 16, 0, 0, 2);
-  if constexpr (NSMAX > 4) {  // NKT = 15: k-tiles 15..29 touch five fragments, one past what a request holds
+  // a request holds four fragments, all that a wave's k-tiles touch but at NKT = 15 (its k-tiles 15..29 touch five)
+  constexpr int FRAGS = NKT % 4 == 0 ? NKT / 4 : NKT % 2 == 0 ? (NKT + 5) / 4 : (NKT + 6) / 4;
+  if constexpr (FRAGS > 4) {
     if (lane < ns * 16 - 64)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(sr, (lds_void_t*)&ssc[wave][256], 16, kgA * 256 + 1024 + lane * 16, 0, 0, 2);
   }

@@ -493,3 +493,14 @@ def test_small_tile_requests_are_as_counted(out, tile, nx, nf, stages):
     full = (stages - 1) * nw + (stages - 2) * nx
     want = [full] * (stages + 1) + [(stages - 1 - i) * (nw + nx) for i in range(1, stages)]
     assert all(w <= x for w, x in zip(waits, want)), (waits, want)
+
+
+@pytest.mark.parametrize("nkt", range(1, 17))
+def test_gemv_row_groups_request_their_scales_once(nkt):
+    """kern_mx_gemv_bf16_r{nkt}: a request brings four scale fragments, and only at nkt = 15 do a wave's k-tiles touch
+    five. In the built code object the non-temporal buffer->LDS requests (the scales') are as many as that needs."""
+    frags = max((w * nkt % 4 + nkt - 1) // 4 + 1 for w in range(4))
+    assert (frags == 5) == (nkt == 15)
+    n = sum(op.startswith("buffer_load") and "lds" in arg and " nt" in arg
+            for _, op, arg in _disassembly(f"kern_mx_gemv_bf16_r{nkt}"))
+    assert n == -(-frags // 4), (n, frags)
