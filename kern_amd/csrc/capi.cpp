@@ -565,17 +565,7 @@ extern "C" int kern_mxfp4_gemv_bf16(const void* x, const void* w, const void* w_
   REQUIRE(x && w && w_sf && y, "mxfp4_gemv_bf16: null buffer");
   const int32_t kg = K / 512, lds_x = 2 * M * K;
   char entry[40];
-  // Row groups (r{K/512}: one workgroup per 16 weight rows, each reading all of x) against the persistent walk
-  // (p{..}: x read once per workgroup, of which there are about 256), by a sweep of both over 8559 launches (M = 1..16,
-  // N = 1024..18432, every K up to 8192, graph replays): the rule is within 1% of the faster one on average.
-  //   M <= 3: row groups at any N (M = 1, N = 2048: 0.71 of the walk's time, N = 18432: 0.94; M = 3 at N > 8192 the
-  //   two are within 5%).
-  //   M > 3: row groups while they all run at once, N <= 4096 per workgroup of their x that a CU's LDS holds, at most
-  //   two (M = 5, N = 3584, K = 7680: 5.4 against 7.7 us), else the walk (M = 8, N = 7168, K = 7680: 9.2 against
-  //   10.1 us; M = 16, N = 8192, K = 2560: 5.8 against 8.5). At K = 512 the walk is ahead from N = 4096 on (M = 16,
-  //   N = 7168: 3.4 against 3.9 us).
-  const bool one_round = N <= 4096 * std::min(2, 163840 / (lds_x + 5120)) && (kg > 1 || N <= 4096);
-  if (kg <= 16 && lds_x <= 144 * 1024 && (M <= 3 || one_round)) {
+  if (kern::gemv_row_groups(M, N, K)) {
     // each wave's x slice (M * K / 2 bytes) in its own LDS region
     Args a;
     a.put(x), a.put(w), a.put(w_sf), a.put(y), a.put(M), a.put(N), a.put(K);

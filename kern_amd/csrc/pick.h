@@ -1,4 +1,4 @@
-// Which kernel a GEMM call launches, from its sizes alone. No HIP in here, so that the rules can be checked on the
+// Which kernel a GEMM or GEMV call launches, from its sizes alone. No HIP in here, so that the rules can be checked on the
 // CPU; kern_amd/manifest.py makes the same choices for the manifest ops.
 #pragma once
 #include <stdint.h>
@@ -19,7 +19,9 @@ inline int64_t walk_half_groups(int64_t m) { return std::min<int64_t>(9, ceil_di
 //   M = 32, m = 9216, k = 7168 12.3, 14.2; M = 16, m = 18432, k = 8192 15.8, 19.6; M = 1, m = 4096, k = 1024 3.4, 3.6;
 //   M = 16, m = 7168, k = 8192 10.1, 9.0; M = 64, m = 4096, k = 4096 9.7, 6.1; M = 64, m = 9216, k = 7168 17.3, 16.6.
 // Past m = 18432 the walk needs a second round of workgroups (M = 2, m = 22528, k = 8192: the tile takes 0.94 of it).
-// By this rule no shape is more than 2.5% slower than by the walk alone.
+// By this rule no shape is more than 2.5% slower than by the walk alone, nor any of 6512 more with every weight from HBM
+// (0.87 of the walk's time on average); with the Infinity Cache full of written lines, whose way out the tiles' cached
+// reads wait for, tiles at m > 6144, k >= 7168 are up to 24% slower (M = 1, m = 8192, k = 7168).
 inline bool takes_walk(int64_t M, int64_t m, int64_t k) {
   if (M > 64 || k % 1024 || m > 18432) return false;
   const int64_t ktw = k / 1024;
@@ -127,6 +129,26 @@ inline const SmallTile8* small_tile8(int64_t m, int64_t n, int64_t k) {
     if (!best || u < us) best = &t, us = u, most = (rounds <= 2 ? 0.85 : 0.72) * large;
   }
   return best && us < most ? best : nullptr;
+}
+
+// The decode GEMV at K <= 8192: row groups (kern_mx_gemv_bf16_r{K/512}: one workgroup per 16 weight rows, each reading
+// all of x into its LDS) or the persistent walk (p{..}: x read once per workgroup, of which there are about 256). Over
+// 1793 shapes (M = 1, 2, 3, 4, 5, 6, 8, 10, 12, 16, eleven N = 1024..18432, every K; graph replays) the choice is within
+// 0.5% of the faster on average.
+//   M <= 3: row groups at any N (M = 1, N = 2048: 0.71 of the walk's time, N = 18432: 0.94). At M = 3, N > 8192 the
+//   walk is ahead at long K (K >= 6144: by 8% on average, 18% at N = 18432, K = 8192; over all K by 2%).
+//   M > 3: row groups while they all run at once, N <= 4096 per workgroup of their LDS that a CU holds, at most two
+//   (M = 5, N = 3584, K = 7680: 5.4 against 7.7 us), else the walk (M = 8, N = 7168, K = 7680: 9.2 against 10.1 us;
+//   M = 16, N = 8192, K = 2560: 5.8 against 8.5; M = 15 there, where one fits: 6.0 against 8.4). At M = 12..16,
+//   N = 6144..8192 and K <= 3072 the walk would still be 10% to 21% ahead (M = 12, N = 8192, K = 3072: 5.6 against
+//   6.8). At K = 512 it is from N = 4096 on (M = 16, N = 7168: 3.4 against 3.9 us).
+// LDS of a row group's workgroup beside x: the waves' sums and (kg + 6) / 4 scale fragments for each wave
+inline int64_t gemv_row_group_lds(int64_t kg) { return 4096 + 1024 * ((kg + 6) / 4); }
+inline bool gemv_row_groups(int64_t M, int64_t N, int64_t K) {
+  const int64_t kg = K / 512, x = 2 * M * K;
+  if (kg > 16 || x > 144 * 1024) return false;
+  if (M <= 3) return true;
+  return N <= 4096 * std::min<int64_t>(2, 163840 / (x + gemv_row_group_lds(kg))) && (kg > 1 || N <= 4096);
 }
 
 }  // namespace kern

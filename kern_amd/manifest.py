@@ -208,14 +208,22 @@ def _rows(rows_var: str) -> dict:
     return {"pack": {"size": 4, "fields": [{"at": 0, "var": rows_var}]}}
 
 
+def gemv_row_groups(M: int, N: int, K: int) -> bool:
+    """Whether the decode GEMV runs one workgroup per row group (csrc/pick.h: gemv_row_groups, the same rule)."""
+    kg, x = K // 512, 2 * M * K
+    if kg > GEMV_MAX_NKT or x > 144 * 1024:
+        return False
+    at_once = 4096 * min(2, 163840 // (x + 4096 + 1024 * ((kg + 6) // 4)))
+    return M <= 3 or (N <= at_once and (kg > 1 or N <= 4096))
+
+
 def _gemv_launch(N: int, K: int, M: int, rows_var: str) -> dict:
     """The launch kern_mxfp4_gemv_bf16 makes for M rows of x [M][K] against weights [N][K/2] (capi.cpp)."""
     kg = K // 512
     params = ["in buffer<bf16>", "in buffer<u8>", "in buffer<u8>", "out buffer<bf16>", "bytes<4>", "i32", "i32"]
     args = [{"param": i} for i in range(4)] + [_rows(rows_var), {"i32": N}, {"i32": K}]
     row_groups = [N // 16, 1, 1]
-    one_round = N <= 4096 * min(2, 163840 // (2 * M * K + 5120)) and (kg > 1 or N <= 4096)
-    if kg <= GEMV_MAX_NKT and 2 * M * K <= 144 * 1024 and (M <= 3 or one_round):
+    if gemv_row_groups(M, N, K):
         # one workgroup per 16-row group, each wave's x slice (2 * M * K bytes in all) in LDS
         return {"entry": f"kern_mx_gemv_bf16_r{kg}", "params": params, "block": [256, 1, 1], "grid": row_groups,
                 "shared_mem": {"mul": [rows_var, 2 * K]}, "args": args}
@@ -227,8 +235,8 @@ def _gemv_launch(N: int, K: int, M: int, rows_var: str) -> dict:
     if kg <= GEMV_MAX_NKT:
         H = N // 8
         hb = min(9, _ceil(H, 256))
-        return {"entry": f"kern_mx_gemv_bf16_p{_ceil(kg, 2)}{'h' if kg % 2 else ''}", "params": params + ["i32"], "block": [512, 1, 1],
-                "grid": [_ceil(H, hb), 1, 1], "args": args + [{"i32": hb}]}
+        return {"entry": f"kern_mx_gemv_bf16_p{_ceil(kg, 2)}{'h' if kg % 2 else ''}", "params": params + ["i32"],
+                "block": [512, 1, 1], "grid": [_ceil(H, hb), 1, 1], "args": args + [{"i32": hb}]}
     # K > 8192: x staged in slices of sb k-tiles per wave, nb k-tiles of weights in flight together
     sb = next(c for c in range(min(kg, GEMV_MAX_ROWS // M), 0, -1) if kg % c == 0)
     nb = next((c for c in (7, 4, 2) if sb % c == 0), 1)

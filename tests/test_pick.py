@@ -4,6 +4,7 @@ there was one to make."""
 import ctypes
 import os
 import random
+import re
 import subprocess
 
 import pytest
@@ -27,6 +28,8 @@ extern "C" int tile8(int64_t m, int64_t n, int64_t k) {
   const SmallTile8* t = small_tile8(m, n, k);
   return t ? t->rows * 1000 + t->weights : 0;
 }
+extern "C" int gemv(int64_t M, int64_t N, int64_t K) { return gemv_row_groups(M, N, K); }
+extern "C" int64_t gemv_lds(int64_t kg, int64_t, int64_t) { return gemv_row_group_lds(kg); }
 extern "C" int64_t ring(int64_t M, int64_t m, int64_t k) { return ring_rows(M, m, k); }
 """
 
@@ -39,8 +42,8 @@ def pick(tmp_path_factory):
     subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", f"-I{csrc}", str(d / "shim.cpp"), "-o",
                     str(d / "shim.so")], check=True)
     L = ctypes.CDLL(str(d / "shim.so"))
-    L.ring.restype = ctypes.c_int64
-    for f in (L.takes, L.ring, L.tile8):
+    L.ring.restype = L.gemv_lds.restype = ctypes.c_int64
+    for f in (L.takes, L.ring, L.tile8, L.gemv, L.gemv_lds):
         f.argtypes = [ctypes.c_int64] * 3
     L.tile.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_void_p] * 3
     return L
@@ -150,6 +153,37 @@ def test_mxfp8_large_tiles_where_they_are_faster(pick, M, N, K, large, tile):
                                          (2048, 2048, 7168, False), (4096, 2048, 7168, False), (300, 520, 2 << 20, False)])
 def test_mxfp8_routes(pick, M, N, K, small):
     assert bool(pick.tile8(M, N, K)) == small
+
+
+def test_gemv_counts_the_row_groups_lds(pick):
+    """The rule's LDS of a row group's workgroup is the code object's static LDS, and its row groups run at once: more
+    than one workgroup a CU only where two fit."""
+    if not os.path.exists(ops.HSACO_PATH):
+        pytest.skip("code object not built")
+    notes = subprocess.run([os.path.join(kb.ROCM, "llvm", "bin", "llvm-readobj"), "--notes", ops.HSACO_PATH],
+                           capture_output=True, text=True, check=True).stdout
+    for kg in range(1, 17):
+        block = re.search(rf"(?:(?!\.name:).)*\.name: +kern_mx_gemv_bf16_r{kg}\n", notes, re.S).group(0)
+        static = int(re.findall(r"\.group_segment_fixed_size: +(\d+)", block)[-1])
+        assert pick.gemv_lds(kg, 0, 0) == static
+        for M in range(4, 17):
+            for N in (16, 4096, 4112, 8192, 8208):
+                if pick.gemv(M, N, 512 * kg):
+                    assert N // 16 <= 256 * (163840 // (2 * M * 512 * kg + static)), (M, N, kg)
+
+
+def test_manifest_makes_the_same_gemv_choice(pick):
+    for M in range(1, 17):
+        for kg in range(1, 18):
+            for N in (16, 4080, 4096, 4112, 8192, 8208, 18432):
+                assert bool(pick.gemv(M, N, 512 * kg)) == mf.gemv_row_groups(M, N, 512 * kg), (M, N, kg)
+
+
+@pytest.mark.parametrize("M,N,K,row_groups", [(5, 8192, 7680, False), (5, 4096, 7680, True), (1, 18432, 7168, True),
+                                              (8, 7168, 7680, False), (15, 8192, 2560, False), (16, 8192, 2560, False),
+                                              (16, 7168, 512, False)])
+def test_gemv_routes(pick, M, N, K, row_groups):
+    assert bool(pick.gemv(M, N, K)) == row_groups
 
 
 @pytest.mark.parametrize("K", [1024, 2048, 4096, 7168, 8192])
