@@ -14,14 +14,14 @@ inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 inline int64_t walk_half_groups(int64_t m) { return std::min<int64_t>(9, ceil_div(m / 8, 256)); }
 
 // Where the walk is taken, else the tiles below. Its waves split K, so it streams wide weights faster; its workgroups
-// each read all of the activations, so more rows and narrow weights favour the tiles. Both measured at 5107 shapes
+// each read all of the activations, so more rows and narrow weights favour the tiles. Both measured at 11619 shapes
 // (M = 1..64, m = 256..24576, weights from HBM and from the Infinity Cache; walk, tile in us):
 //   M = 32, m = 9216, k = 7168 12.3, 14.2; M = 16, m = 18432, k = 8192 15.8, 19.6; M = 1, m = 4096, k = 1024 3.4, 3.6;
 //   M = 16, m = 7168, k = 8192 10.1, 9.0; M = 64, m = 4096, k = 4096 9.7, 6.1; M = 64, m = 9216, k = 7168 17.3, 16.6.
 // Past m = 18432 the walk needs a second round of workgroups (M = 2, m = 22528, k = 8192: the tile takes 0.94 of it).
-// By this rule no shape is more than 2.5% slower than by the walk alone, nor any of 6512 more with every weight from HBM
-// (0.87 of the walk's time on average); with the Infinity Cache full of written lines, whose way out the tiles' cached
-// reads wait for, tiles at m > 6144, k >= 7168 are up to 24% slower (M = 1, m = 8192, k = 7168).
+// By this rule none of them is more than 2.5% slower than by the walk alone, and the mean is 0.87 of it. Only right
+// behind 768 MB of writes, the weights from HBM, are tiles slower than the walk at m > 6144, k >= 7168, up to 24%
+// (M = 1, m = 8192, k = 7168).
 inline bool takes_walk(int64_t M, int64_t m, int64_t k) {
   if (M > 64 || k % 1024 || m > 18432) return false;
   const int64_t ktw = k / 1024;

@@ -163,8 +163,9 @@ def test_gemm_closed_form_kat(ops):
 # --------------------------------------------------------------------------------------- dense e4m3 (config 3 mode)
 
 # small M (one live 16-row subtile, or one and a row), ragged M, K not a multiple of 1024; the last 128-row
-# tile of 20, 40, 70, 90, 100 and 120 rows: the activation loader's six (live subtiles, live 32-row
-# request blocks) cases, (0, 1) (0, 2) (1, 3) (2, 3) (3, 4) (4, 4) for its rows 64-127
+# tile of 20, 40, 70, 90, 100 and 120 rows: the ring's activation loader's six (live subtiles, live 32-row
+# request blocks) cases, (0, 1) (0, 2) (1, 3) (2, 3) (3, 4) (4, 4) for its rows 64-127. The entry takes the ring
+# for the 4096 rows and small tiles for the rest; test_gpu_large_tiles.py runs these on the ring by name
 @pytest.mark.parametrize("M,m,k", [(300, 512, 1024), (4096, 2048, 7168), (5, 512, 1024), (16, 2048, 7168),
                                    (17, 512, 1536), (148, 512, 1024), (168, 512, 1024), (198, 512, 1024),
                                    (218, 512, 1024), (228, 512, 1024), (248, 512, 1024)])
@@ -659,7 +660,8 @@ def test_mxfp8_gemm_kat(ops):
     np.testing.assert_array_equal(to_np(out), wl.f32_to_bf16_bits(mxfp8_kat(-1)["want"]))
 
 
-# ragged m, n and k; and the benchmark's shape, config 3's 4096 x 2048 x 7168
+# ragged m, n and k (small tiles; test_gpu_large_tiles.py has them on kern_mx_gemm_mxfp8); and the benchmark's shape,
+# config 3's 4096 x 2048 x 7168
 @pytest.mark.parametrize("m,n,k", [(300, 520, 1024), (64, 1000, 2080), (200, 256, 96), (2048, 2048, 7168),
                                    (4096, 2048, 7168)])
 def test_mxfp8_gemm_random(ops, oracle, m, n, k):
@@ -719,7 +721,7 @@ class _HighArena:
 
 def test_ring_operands_above_bit31(ops, oracle):
     """The LDS-ring GEMMs with every operand and output at an address whose bit 31 is set: the config-3 mode
-    GEMM, FC1 and FC2 (slots of 20..128 rows, all on the ring) each equal the same launch on ordinary buffers
+    GEMM (a small tile by the entry's choice; test_gpu_large_tiles.py launches the ring), FC1 and FC2 (slots of 20..128 rows, all on the ring) each equal the same launch on ordinary buffers
     bit for bit; those are checked against the oracle here too (the GEMM's accumulators, FC1's codes through
     its debug twin, FC2's rows)."""
     from tests import _moe

@@ -4,8 +4,9 @@
 
 Each tile runs at its edges: one row, one row short of a whole tile, one past it; K from one k group of 512 to past two
 rounds of its stages, every remainder among them; fewer and more tiles than the eight XCDs. The ring kernel is compared
-with the CPU oracle in test_gpu_stack.py and test_gpu_sweep.py; here the entry as the C ABI picks it is as well, on both
-sides of a switch and where it takes the ring for some rows and small tiles for the rest.
+with the CPU oracle, by name, in test_gpu_large_tiles.py; here the entries as the C ABI picks them are as well, the walk
+over wide weights is, and a launch that takes the ring for some rows and small tiles for the rest has the ring's bits
+(test_pick.py holds which shapes those are).
 """
 import numpy as np
 import pytest
@@ -70,7 +71,7 @@ def test_tiles_have_the_rings_bits(ops, rows, weights, waves, stages):
 @pytest.mark.parametrize("M,N,K", [(16, 256, 512), (100, 512, 1024), (130, 768, 1536), (40, 6144, 3584),
                                    (1100, 8192, 512), (1540, 5632, 512)])
 def test_dense_gemm_as_picked(ops, oracle, M, N, K):
-    """Against the oracle; (1540, 5632, 512) has 286 ring tiles, so rows past the ring's first round may go to small tiles."""
+    """Against the oracle, small tiles or (the last two, 288 and 286 ring tiles) the ring by the entry's choice."""
     print(f"[dense] M={M} N={N} K={K}", flush=True)
     w, s, q, qs = _operands(ops, M, N, K, 60)
     c = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")

@@ -6,7 +6,7 @@
   rounding of the kernel's own accumulators, bit for bit.
 * Layers of the stack (quantize -> QKV -> O -> quantize + routing -> MoE of 256 experts, top-8, H = 7168,
   I = 2048 -> RMS finalize), chained as the bench's step chains them, at M = 1 (decode GEMV for QKV and O;
-  two layers), M = 64 (quantizer + dense walk; two layers) and M = 2048 (quantizer + tiled GEMM, 16,384
+  two layers), M = 64 (quantizer + dense GEMMs; two layers) and M = 2048 (quantizer + ring GEMMs, 16,384
   routed rows; one layer), captured once through the library's own hipGraph C ABI (kern_graph_begin / end)
   and replayed: every replay equals the eager run bit for bit, and every stage of every layer is checked
   against the oracle on the GPU's own inputs to that stage (quantizers and routing tables bit-exact, GEMV /
@@ -37,11 +37,9 @@ def ops():
     return ops
 
 
-# kern_mxfp4_gemm_bf16 takes the persistent walk (kern_mx_gemm_bf16_s{k/1024}) at M <= 64 with k = 1024 *
-# {1, 2, 4, 7, 8} (config 5's M = 64), else the tiled GEMM (config 5's M = 2048). The cases reach every
-# persistent instance with ragged token groups (M = 1, 17, 33, 50), half-group shares of 1, 2, 3 and 9
-# with a ragged last workgroup (m = 4352: 544 half groups in shares of 3), and the tiled side of both
-# bounds (M = 65; k = 3072).
+# What kern_mxfp4_gemm_bf16 launches here (csrc/pick.h): the walk (kern_mx_gemm_bf16_s{k/1024}) for (64, QKV, H) and
+# (64, 18432, 7168), half-group shares of 5 and 9; the ring for M = 2048; small tiles for the rest, with ragged token
+# rows (M = 1, 17, 33, 50, 65, 40). tests/test_gpu_small_tiles.py takes every walk instance and every tile.
 @pytest.mark.parametrize("M,m,k", [(64, QKV, H), (64, H, OIN), (2048, QKV, H), (2048, H, OIN),
                                    (17, 256, 1024), (33, 4352, 2048), (50, 2304, 4096), (1, 512, 8192),
                                    (64, 18432, 7168), (65, 2304, 4096), (40, 768, 3072)])
@@ -69,8 +67,8 @@ def test_gemm_bf16_config5_shapes(ops, oracle, M, m, k):
 # Layers chained as bench.py's config-5 step runs them: layer l's QKV input is layer l-1's finalize output;
 # the O input stands in for attention; O's output goes through moe_quant_routing (the quantizer and the
 # routing tables in one call) into production FC1 (no debug output), FC2 and the RMS finalize. M = 1 takes
-# the decode GEMV for QKV and O, M = 64 the dense walk, M = 2048 the tiled GEMM and a MoE of 16,384 routed
-# rows (64 per expert: every slot on the LDS ring with its second wave group idle).
+# the decode GEMV for QKV and O, M = 64 the dense walk for QKV and a small tile for O, M = 2048 the ring and a
+# MoE of 16,384 routed rows (64 per expert: every slot on the LDS ring with its second wave group idle).
 @pytest.mark.parametrize("M,NL", [(1, 2), (64, 2), (2048, 1)])
 def test_config5_layers_graph(ops, oracle, M, NL):
     print(f"[config 5] M={M}, {NL} layer(s): weights", flush=True)

@@ -3,8 +3,8 @@
 * kern_mxfp4_gemv_bf16 (W4A16 decode): M in 1..16, N a multiple of 16 from 16 to 19200 (ragged shares of
   the persistent kernel's half groups), K from 512 to 16384 (every kernel the entry picks: the row-group
   instances, the k-group loop, the persistent instances and the sliced kernel).
-* kern_mxfp4_gemm_bf16 (dense bf16 out): M in 1..80 (the persistent walk up to 64, tiled above), m a
-  multiple of 256, k in {1024, 2048, 3072, 4096, 7168, 8192}; the bf16 output is the RNE rounding of the
+* kern_mxfp4_gemm_bf16 (dense bf16 out): M in 1..80 (small tiles, and the walk over wide weights; the ring
+  kernel gets half of these shapes by name in test_gpu_large_tiles.py), m a multiple of 256, k in {1024, 2048, 3072, 4096, 7168, 8192}; the bf16 output is the RNE rounding of the
   kernel's own f32 sums, and those sums are within the north-star tolerance of the oracle.
 
 The shapes come from a fixed seed, so each run sends the same sequence of launches; kernels that read

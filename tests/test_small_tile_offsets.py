@@ -1,4 +1,4 @@
-"""The scalar offsets of the small tiles' memory requests, from the built code objects, on the CPU.
+"""The small tiles' memory requests, from the built code objects, on the CPU: scalar offsets, and hand-counted waits.
 
 A buffer request's range check compares the lane's offset with the resource's length minus the request's scalar offset.
 That difference may not wrap: a scalar offset past the length (a negative one among them) would let lanes through that
@@ -34,7 +34,7 @@ class Wave:
     one known value in all lanes."""
 
     def __init__(self, kernarg, workgroup, wave):
-        self.kernarg, self.vcc, self.scc, self.requests = kernarg, None, 0, []
+        self.kernarg, self.vcc, self.scc, self.requests, self.events = kernarg, None, 0, [], []
         self.s = {0: 0x100000, 1: 0, 2: workgroup[0], 3: workgroup[1]}
         self.v, self.tid0 = {}, 64 * wave
 
@@ -83,6 +83,10 @@ class Wave:
             return self.put(d, None, wide)
         top = M64 if wide else M32
         sa, sb = (_s32(a), _s32(b)) if not wide else (a, b)
+        if name == "bfe":  # a field: offset and width; signed, its top bit is its sign
+            width = b >> 16 & 127
+            f = a >> (b & 31) & ((1 << width) - 1)
+            a, b, name = f - (1 << width if ty == "i32" and width and f >> (width - 1) else 0), 0, "or"
         carry = self.scc if name == "addc" else 0
         v = {"mov": a, "add": a + b, "addc": a + b + (carry or 0), "sub": a - b, "mul": a * b, "and": a & b, "or": a | b,
              "xor": a ^ b, "andn2": a & ~b, "lshl": a << (b & (63 if wide else 31)), "lshr": a >> (b & 31),
@@ -130,18 +134,20 @@ class Wave:
                 for i in range(n):
                     self.v[r + i] = None if v is None else v & M32
 
-    def run(self, ins, limit=200000):
+    def run(self, ins, stop=None, limit=200000):
+        """Steps to the end of the program, or to the first `stop` instruction; the requests as (address, scalar offset,
+        resource length)."""
         at = {a: i for i, (a, _, _) in enumerate(ins)}
         i = 0
         for _ in range(limit):
             a, op, arg = ins[i]
             args = [t.strip() for t in arg.split("<")[0].split(",")]
             i += 1
-            if op == "s_endpgm":
+            if op in ("s_endpgm", stop):
                 return self.requests
             if op.startswith(("s_branch", "s_cbranch")):
                 k = int(args[0])
-                taken = {"s_branch": 1, "s_cbranch_scc1": self.scc, "s_cbranch_execz": 0, "s_cbranch_vccnz": self.vcc,
+                taken = {"s_branch": 1, "s_cbranch_scc1": self.scc, "s_cbranch_execz": 0, "s_cbranch_execnz": 1, "s_cbranch_vccnz": self.vcc,
                          "s_cbranch_vccz": None if self.vcc is None else self.vcc == 0,
                          "s_cbranch_scc0": None if self.scc is None else not self.scc}[op]
                 assert taken is not None, f"{op} at {a:#x} on an unknown value"
@@ -151,7 +157,17 @@ class Wave:
                 self.load(*args)
             elif op.startswith("s_cmp"):
                 self.cmp(op, *args)
+            elif op.startswith("s_bitcmp"):
+                v = self.get(args[0])
+                self.scc = None if v is None else int(v >> (self.get(args[1]) & 31) & 1 == int(op[8]))
+            elif op == "s_waitcnt":
+                for c in ("vmcnt", "lgkmcnt"):
+                    if m := re.search(rf"{c}\((\d+)\)", arg):
+                        self.events.append((c, int(m.group(1))))
+            elif op.startswith(("ds_read", "global_")):
+                self.events.append((op,))
             elif op.startswith(("buffer_load", "buffer_store")):
+                self.events.append(("lds_request" if arg.endswith("lds") else op,))
                 srsrc, soff = [t for t in args if t.startswith("s[")][0], arg.split(" offen")[0].split(",")[-1].strip()
                 r, _ = self.regs(srsrc)
                 self.requests.append((a, self.get(soff), self.s.get(r + 2)))
@@ -160,7 +176,7 @@ class Wave:
             elif op.startswith("s_and_saveexec"):
                 self.put(args[0], None, True)
                 self.scc = None
-            elif op.startswith("s_") and not op.startswith(("s_nop", "s_waitcnt", "s_barrier")):
+            elif op.startswith("s_") and op not in ("s_nop", "s_barrier"):
                 self.alu(op, *args)
         raise AssertionError("no end within the limit")
 
@@ -190,3 +206,56 @@ def test_scalar_offsets_stay_within_the_resources(out, tile, waves, stages):
                     assert soff is not None and n is not None, hex(a)
                     assert soff <= n, (f"request at {a:#x}: scalar offset {_s32(soff)} with {n} bytes "
                                        f"(K = {K}, workgroup {workgroup}, wave {wave})")
+
+
+def _check_mxfp8_waits(ins, tile, ktiles):
+    rows, weights = map(int, tile.split("x"))
+    mt, ng = rows // 16, weights // 16
+    M, N, K = 2 * rows, 2 * weights, 128 * ktiles - 32
+    kernarg = struct.pack("<5Q4i3I", *[0x200000000000 + (i << 34) for i in range(5)], M, N, K, N, 2, 2, 1)
+    for wave in range(8):
+        w = Wave(kernarg + bytes(64), (1, 1), wave)
+        for a, soff, n in w.run(ins, stop="s_barrier"):
+            assert soff is not None and n is not None and soff <= n, hex(a)
+        steps = (ktiles - wave + 7) // 8
+        out, sent, arrived, reads, unread, step = [], 0, 0, 0, False, 0
+        for e in w.events:
+            if e[0] == "lds_request":
+                assert not unread, f"wave {wave}: a request while step {step}'s reads are outstanding"
+                # a slot's refill comes after its step's reads
+                assert sent // (2 * mt) < 2 or reads >= (sent // (2 * mt) - 2) * 2 * (mt + ng) + 2 * mt
+                out.append(True)
+                sent += 1
+            elif e[0].startswith(("buffer_", "global_")):
+                out.append(False)
+            elif e[0] == "vmcnt":
+                while len(out) > e[1]:
+                    arrived += out.pop(0)
+            elif e[0] == "lgkmcnt" and e[1] == 0:
+                unread = False
+            elif e[0].startswith("ds_read"):
+                step, at = divmod(reads, 2 * (mt + ng))  # 2 mt reads of activations, then 2 ng of weights
+                if at < 2 * mt:
+                    assert arrived >= 2 * mt * (step + 1), f"wave {wave}: step {step} of {steps} reads ahead of its wait"
+                    unread = True
+                reads += 1
+        assert reads == 2 * (mt + ng) * steps and sent == arrived == 2 * mt * steps
+
+
+@pytest.mark.parametrize("tile", ["16x16", "16x32", "16x64", "32x64", "32x128", "48x64", "64x64"])
+def test_mxfp8_tiles_wait_for_their_activations(tile):
+    """A wave of kern_mx_gemm_mxfp8_t* takes every eighth k-tile and has two k-tiles of activations on their way into its
+    LDS, waited for by a count that depends on the step (first, last, both, neither). Its instructions as they execute,
+    up to the barrier at which the waves add their sums: when a k-tile's activations are read, the requests that brought
+    them have retired; a request into a slot follows a full wait for the slot's reads; none is left in flight; and scalar
+    offsets stay within the resources. With none to five k-tiles a wave; a wait that is one too large is caught."""
+    ins = _disassembly(f"kern_mx_gemm_mxfp8_t{tile}")
+    for ktiles in (1, 8, 9, 16, 17, 24, 25, 33, 41):
+        _check_mxfp8_waits(ins, tile, ktiles)
+    rows, weights = map(int, tile.split("x"))
+    first = f"vmcnt({weights // 8 + rows // 8})"  # the first step's, behind it the next k-tile's requests and the weights'
+    late = [(a, op, arg.replace(first, f"vmcnt({weights // 8 + rows // 8 + 1})") if op == "s_waitcnt" else arg)
+            for a, op, arg in ins]
+    assert late != ins
+    with pytest.raises(AssertionError, match="ahead of its wait"):
+        _check_mxfp8_waits(late, tile, 17)
