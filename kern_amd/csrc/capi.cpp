@@ -492,7 +492,7 @@ namespace {
 
 using kern::SmallTile;
 struct DenseGemm {
-  const char* ring;  // the ring's entry; a small tile's is this + _t{rows}x{weights}
+  const char* ring;  // the ring's entry
   const uint8_t *a, *sf_a, *b, *sf_b;
   uint8_t* c;
   int out_bytes;
@@ -508,18 +508,15 @@ int launch_dense(const DenseGemm& G, int64_t r0, int32_t rows, const SmallTile* 
   if (G.d_scale) a.put(G.d_scale);
   a.put(rows), a.put(G.m), a.put(G.k), a.put(G.dbg ? G.dbg + r0 * G.m : nullptr);
   if (!t) return launch(G.ring, (uint32_t)(G.m / 256), (uint32_t)((rows + 127) / 128), 1, kBmmThreads, stream, a);
-  char entry[64];
-  snprintf(entry, sizeof entry, "%s_t%dx%d", G.ring, t->rows, t->weights);
-  return launch(entry, (uint32_t)((G.m + t->weights - 1) / t->weights), (uint32_t)((rows + t->rows - 1) / t->rows), 1,
+  return launch(G.d_scale ? t->e4m3 : t->bf16, (uint32_t)((G.m + t->weights - 1) / t->weights), (uint32_t)((rows + t->rows - 1) / t->rows), 1,
                 64u * (uint32_t)t->waves, stream, a, (uint32_t)kern::small_tile_lds(*t, G.k));
 }
 int dense_gemm(const DenseGemm& G, int32_t M, void* stream) {
-  const int32_t ring = (int32_t)kern::ring_rows(M, G.m, G.k);
+  const kern::DensePlan p = kern::dense_plan(M, G.m, G.k);
+  const int32_t ring = (int32_t)p.ring_rows;
   if (ring > 0)
     if (int rc = launch_dense(G, 0, ring, nullptr, stream)) return rc;
-  if (ring == M) return KERN_OK;
-  double us = 0;
-  return launch_dense(G, ring, M - ring, kern::best_small_tile(M - ring, G.m, G.k, &us), stream);
+  return ring == M ? KERN_OK : launch_dense(G, ring, M - ring, p.tile, stream);
 }
 
 }  // namespace
@@ -546,12 +543,13 @@ extern "C" int kern_mxfp4_gemm_bf16(const void* a_, const void* sf_a, const void
           M, k);
   if (M == 0) return KERN_OK;
   if (kern::takes_walk(M, m, k)) {
+    static const char* const walk[9] = {nullptr, "kern_mx_gemm_bf16_s1", "kern_mx_gemm_bf16_s2", nullptr,
+                                        "kern_mx_gemm_bf16_s4", nullptr, nullptr, "kern_mx_gemm_bf16_s7",
+                                        "kern_mx_gemm_bf16_s8"};
     const int32_t hb = (int32_t)kern::walk_half_groups(m);
-    char entry[40];
-    snprintf(entry, sizeof entry, "kern_mx_gemm_bf16_s%d", k / 1024);
     Args a;
     a.put(a_), a.put(sf_a), a.put(b), a.put(sf_b), a.put(c), a.put(dbg), a.put(M), a.put(m), a.put(k), a.put(hb);
-    return launch(entry, (uint32_t)((m / 8 + hb - 1) / hb), 1, 1, 512, stream, a);
+    return launch(walk[k / 1024], (uint32_t)((m / 8 + hb - 1) / hb), 1, 1, 512, stream, a);
   }
   return dense_gemm({"kern_mx_gemm_bf16", (const uint8_t*)a_, (const uint8_t*)sf_a, (const uint8_t*)b,
                      (const uint8_t*)sf_b, (uint8_t*)c, 2, nullptr, dbg, m, k},
@@ -564,13 +562,21 @@ extern "C" int kern_mxfp4_gemv_bf16(const void* x, const void* w, const void* w_
           "mxfp4_gemv_bf16: need 1 <= M <= 16, N %% 16 == 0, K %% 512 == 0, K <= 16384 (M=%d N=%d K=%d)", M, N, K);
   REQUIRE(x && w && w_sf && y, "mxfp4_gemv_bf16: null buffer");
   const int32_t kg = K / 512, lds_x = 2 * M * K;
-  char entry[40];
+#define KERN_GEMV(P, S) "kern_mx_gemv_bf16_" #P #S
+#define KERN_GEMV_H(S) KERN_GEMV(p, S##h), KERN_GEMV(p, S)
+  static const char* const rows[16] = {KERN_GEMV(r, 1),  KERN_GEMV(r, 2),  KERN_GEMV(r, 3),  KERN_GEMV(r, 4),
+                                       KERN_GEMV(r, 5),  KERN_GEMV(r, 6),  KERN_GEMV(r, 7),  KERN_GEMV(r, 8),
+                                       KERN_GEMV(r, 9),  KERN_GEMV(r, 10), KERN_GEMV(r, 11), KERN_GEMV(r, 12),
+                                       KERN_GEMV(r, 13), KERN_GEMV(r, 14), KERN_GEMV(r, 15), KERN_GEMV(r, 16)};
+  static const char* const walk[16] = {KERN_GEMV_H(1), KERN_GEMV_H(2), KERN_GEMV_H(3), KERN_GEMV_H(4),
+                                       KERN_GEMV_H(5), KERN_GEMV_H(6), KERN_GEMV_H(7), KERN_GEMV_H(8)};
+#undef KERN_GEMV_H
+#undef KERN_GEMV
   if (kern::gemv_row_groups(M, N, K)) {
     // each wave's x slice (M * K / 2 bytes) in its own LDS region
     Args a;
     a.put(x), a.put(w), a.put(w_sf), a.put(y), a.put(M), a.put(N), a.put(K);
-    snprintf(entry, sizeof entry, "kern_mx_gemv_bf16_r%d", kg);
-    return launch(entry, (uint32_t)(N / 16), 1, 1, 256, stream, a, (uint32_t)lds_x);
+    return launch(rows[kg - 1], (uint32_t)(N / 16), 1, 1, 256, stream, a, (uint32_t)lds_x);
   }
   if (M <= 2) {
     // K > 8192: the same, each wave owning whole 512-wide k groups (a floor or ceiling of KG/4) in a loop,
@@ -588,8 +594,7 @@ extern "C" int kern_mxfp4_gemv_bf16(const void* x, const void* w, const void* w_
     const int32_t hb = std::min<int32_t>(9, (H + 255) / 256);
     Args a;
     a.put(x), a.put(w), a.put(w_sf), a.put(y), a.put(M), a.put(N), a.put(K), a.put(hb);
-    snprintf(entry, sizeof entry, "kern_mx_gemv_bf16_p%d%s", (kg + 1) / 2, kg % 2 ? "h" : "");
-    return launch(entry, (uint32_t)((H + hb - 1) / hb), 1, 1, 512, stream, a);
+    return launch(walk[kg - 1], (uint32_t)((H + hb - 1) / hb), 1, 1, 512, stream, a);
   }
   // K > 8192 at M > 2: one workgroup per row group, x staged per workgroup in slices
   // sb: k-tiles per wave whose slice of x is staged in LDS at once (at most four 16-byte pieces per lane,
@@ -668,10 +673,8 @@ extern "C" int kern_mxfp8_gemm_bf16(const void* a, const void* w, void* c, const
   Args x;
   x.put(a), x.put(w), x.put(c), x.put(a_sf), x.put(w_sf), x.put(m), x.put(n), x.put(k), x.put(ldc);
   if (const kern::SmallTile8* t = kern::small_tile8(m, n, k)) {
-    char entry[64];
-    snprintf(entry, sizeof entry, "kern_mx_gemm_mxfp8_t%dx%d", t->rows, t->weights);
     const uint32_t mt = (uint32_t)t->rows / 16, ng = (uint32_t)t->weights / 16;
-    return launch(entry, (uint32_t)((n + t->weights - 1) / t->weights), (uint32_t)((m + t->rows - 1) / t->rows), 1, 512,
+    return launch(t->entry, (uint32_t)((n + t->weights - 1) / t->weights), (uint32_t)((m + t->rows - 1) / t->rows), 1, 512,
                   stream, x, std::max(8 * (mt + 1) * 4096, 8 * mt * ng * 1024));
   }
   return launch("kern_mx_gemm_mxfp8", (uint32_t)((n + 255) / 256), (uint32_t)((m + 127) / 128), 1, 512, stream, x);

@@ -7,7 +7,11 @@
 
 namespace kern {
 
-inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+// quotients that fit 32 bits are taken there (these rules run before every launch, and 64-bit division is slow)
+inline int64_t ceil_div(int64_t a, int64_t b) {
+  const int64_t n = a + b - 1;
+  return (n | b) >> 32 ? n / b : (int64_t)((uint32_t)n / (uint32_t)b);
+}
 
 // The walk over the weights (kern_mx_gemm_bf16_s{k / 1024}, M <= 64, k = 1024 * {1, 2, 4, 7, 8}): about 256 workgroups
 // of 8 waves with at most nine half groups of 8 weight rows each.
@@ -38,11 +42,16 @@ inline bool takes_walk(int64_t M, int64_t m, int64_t k) {
 // ring's 128 x 256 tiles. All of these accumulate K in the same order, so the choice does not show in the results.
 struct SmallTile {
   int rows, weights, waves, stages;
+  const char *bf16, *e4m3;  // its entries
 };
+#define KERN_SMALL_TILE(R, W, WAVES, STAGES) \
+  {R, W, WAVES, STAGES, "kern_mx_gemm_bf16_t" #R "x" #W, "kern_mx_gemm_e4m3_t" #R "x" #W}
 static const SmallTile kSmallTiles[] = {
-    {16, 32, 2, 8}, {16, 64, 4, 8}, {16, 128, 8, 4}, {32, 128, 8, 4}, {48, 128, 8, 4},
-    {80, 128, 8, 3}, {32, 256, 8, 3}, {48, 256, 8, 3}, {64, 256, 8, 3},
+    KERN_SMALL_TILE(16, 32, 2, 8),  KERN_SMALL_TILE(16, 64, 4, 8),  KERN_SMALL_TILE(16, 128, 8, 4),
+    KERN_SMALL_TILE(32, 128, 8, 4), KERN_SMALL_TILE(48, 128, 8, 4), KERN_SMALL_TILE(80, 128, 8, 3),
+    KERN_SMALL_TILE(32, 256, 8, 3), KERN_SMALL_TILE(48, 256, 8, 3), KERN_SMALL_TILE(64, 256, 8, 3),
 };
+#undef KERN_SMALL_TILE
 // dynamic LDS of a small tile: the activation ring, then the token scales in whole KiB
 inline int64_t small_tile_lds(const SmallTile& t, int64_t k) {
   return (int64_t)t.stages * t.rows * 512 + ceil_div(t.rows * (k / 512 + 1), 64) * 1024;
@@ -91,16 +100,21 @@ inline const SmallTile* best_small_tile(int64_t M, int64_t m, int64_t k, double*
 // 3% to 27% shorter measured and 13% on average (M = 1024, N = 9216, K = 7168, 288 tiles: 70.7 -> 59.3 us). With 5%
 // asked for it was 124 times, up to 14% slower (M = 531, N = 13312, K = 10240), and level at M = 2048, N = 9216,
 // K = 7168 (2.25 rounds).
-inline int64_t ring_rows(int64_t M, int64_t m, int64_t k) {
+struct DensePlan {
+  int64_t ring_rows;
+  const SmallTile* tile;  // for the rest of the rows, if any
+};
+inline DensePlan dense_plan(int64_t M, int64_t m, int64_t k) {
   double us = 0, rest_us = 0;
   const double ring = ring_us(M, m, k);
-  if (best_small_tile(M, m, k, &us) && us < 0.9 * ring) return 0;
+  const SmallTile* tile = best_small_tile(M, m, k, &us);
+  if (tile && us < 0.9 * ring) return {0, tile};
   const int64_t nb = m / 256, rounds = ceil_div(ceil_div(M, 128) * nb, 256);
   const int64_t blocks = 256 * (rounds - 1) / nb;  // whole blocks in all rounds but the last
-  if (blocks > 0 && best_small_tile(M - 128 * blocks, m, k, &rest_us) &&
+  if (blocks > 0 && (tile = best_small_tile(M - 128 * blocks, m, k, &rest_us)) &&
       ring_us(128 * blocks, m, k) + rest_us < 0.87 * ring)
-    return 128 * blocks;
-  return M;
+    return {128 * blocks, tile};
+  return {M, nullptr};
 }
 
 // Small tiles of the MXFP8 x MXFP8 GEMM (kern_mx_gemm_mxfp8_t{rows}x{weights}); the fit of their times and of
@@ -112,8 +126,15 @@ inline int64_t ring_rows(int64_t M, int64_t m, int64_t k) {
 // and never slower than the large tiles; with 15% at any number of rounds 16 were, by up to 24%.
 struct SmallTile8 {
   int rows, weights;
+  const char* entry;
 };
-static const SmallTile8 kSmallTiles8[] = {{16, 16}, {16, 32}, {16, 64}, {32, 64}, {32, 128}, {48, 64}, {64, 64}};
+#define KERN_SMALL_TILE8(R, W) \
+  { R, W, "kern_mx_gemm_mxfp8_t" #R "x" #W }
+static const SmallTile8 kSmallTiles8[] = {
+    KERN_SMALL_TILE8(16, 16),  KERN_SMALL_TILE8(16, 32), KERN_SMALL_TILE8(16, 64), KERN_SMALL_TILE8(32, 64),
+    KERN_SMALL_TILE8(32, 128), KERN_SMALL_TILE8(48, 64), KERN_SMALL_TILE8(64, 64),
+};
+#undef KERN_SMALL_TILE8
 inline const SmallTile8* small_tile8(int64_t m, int64_t n, int64_t k) {
   const int64_t kt = ceil_div(k, 128), big = ceil_div(m, 128) * ceil_div(n, 256);
   const double large =

@@ -28,9 +28,14 @@ extern "C" int tile8(int64_t m, int64_t n, int64_t k) {
   const SmallTile8* t = small_tile8(m, n, k);
   return t ? t->rows * 1000 + t->weights : 0;
 }
+extern "C" const char* entry(int i, int kind) {
+  if (kind == 2) return i < (int)(sizeof kSmallTiles8 / sizeof *kSmallTiles8) ? kSmallTiles8[i].entry : nullptr;
+  if (i >= (int)(sizeof kSmallTiles / sizeof *kSmallTiles)) return nullptr;
+  return kind ? kSmallTiles[i].e4m3 : kSmallTiles[i].bf16;
+}
 extern "C" int gemv(int64_t M, int64_t N, int64_t K) { return gemv_row_groups(M, N, K); }
 extern "C" int64_t gemv_lds(int64_t kg, int64_t, int64_t) { return gemv_row_group_lds(kg); }
-extern "C" int64_t ring(int64_t M, int64_t m, int64_t k) { return ring_rows(M, m, k); }
+extern "C" int64_t ring(int64_t M, int64_t m, int64_t k) { return dense_plan(M, m, k).ring_rows; }
 """
 
 
@@ -61,6 +66,16 @@ def dense_route(pick, M, N, K, out="bf16"):
         return "walk"
     ring = pick.ring(M, N, K)
     return "ring" if ring == M else "split" if ring else "t%dx%d" % tile_of(pick, M, N, K)[:2]
+
+
+def test_every_tile_has_an_entry(pick):
+    pick.entry.restype = ctypes.c_char_p
+    for kind, prefix in enumerate(("kern_mx_gemm_bf16_t", "kern_mx_gemm_e4m3_t", "kern_mx_gemm_mxfp8_t")):
+        got, i = set(), 0
+        while e := pick.entry(i, kind):
+            got.add(e.decode())
+            i += 1
+        assert got == {e for e in kb.ENTRIES if e.startswith(prefix)}
 
 
 def test_manifest_makes_the_same_dense_choice(pick):
