@@ -664,9 +664,9 @@ GEMV_PERSISTENT(8h, 8, true)
 // once. Requested straight in operand pieces, each request gathered 16 rows (M = 64, N = 9216: 25.8
 // against 17.0 us). Both scale operands arrive shifted to byte 0 (OPSEL 0). The eight partial sums meet
 // in LDS one token group at a time; dbg (if not null) receives the f32 sums the bf16 values round.
-// Taken (kern_mxfp4_gemm_bf16) for wide weights, N > 8192 at most M: its waves hold different parts of K, so its
-// requests are spread over memory where the small tiles' stay in step (gemm_tiles; M = 32, N = 9216, K = 7168: 12.3
-// against their 14.2 us; M = 16, N = 18432, K = 8192: 15.8 against 19.6).
+// Taken (kern_mxfp4_gemm_bf16) for wide weights, N > 8192 at K >= 7168: its waves split K, so a workgroup asks for
+// eight times as many parts of memory at once as one of gemm_tiles (M = 32, N = 9216, K = 7168: 13.0 against 14.4 us;
+// M = 16, N = 18432, K = 8192: 17.3 against 19.7, every weight from HBM).
 template <int KTW>
 KERN_DEV void gemm_skinny_bf16(const uint8_t* __restrict__ w, const uint8_t* __restrict__ wsf,
                                const uint8_t* __restrict__ xq, const uint8_t* __restrict__ xsf,

@@ -17,24 +17,22 @@ inline int64_t ceil_div(int64_t a, int64_t b) {
 // of 8 waves with at most nine half groups of 8 weight rows each.
 inline int64_t walk_half_groups(int64_t m) { return std::min<int64_t>(9, ceil_div(m / 8, 256)); }
 
-// Where the walk is taken, else the tiles below. Its waves split K, so it streams wide weights faster; its workgroups
-// each read all of the activations, so more rows and narrow weights favour the tiles. Both measured at 11619 shapes
-// (M = 1..64, m = 256..24576, weights from HBM and from the Infinity Cache; walk, tile in us):
-//   M = 32, m = 9216, k = 7168 12.3, 14.2; M = 16, m = 18432, k = 8192 15.8, 19.6; M = 1, m = 4096, k = 1024 3.4, 3.6;
-//   M = 16, m = 7168, k = 8192 10.1, 9.0; M = 64, m = 4096, k = 4096 9.7, 6.1; M = 64, m = 9216, k = 7168 17.3, 16.6.
-// Past m = 18432 the walk needs a second round of workgroups (M = 2, m = 22528, k = 8192: the tile takes 0.94 of it).
-// By this rule none of them is more than 2.5% slower than by the walk alone, and the mean is 0.87 of it. Only right
-// behind 768 MB of writes, the weights from HBM, are tiles slower than the walk at m > 6144, k >= 7168, up to 24%
-// (M = 1, m = 8192, k = 7168).
+// Where the walk is taken, else the tiles below. Its waves split K, so it streams wide weights from HBM faster; its
+// workgroups each read all of the activations, so more rows and narrow weights favour the tiles. Walk, tile in us:
+//   M = 32, m = 9216, k = 7168 13.0, 14.4; M = 16, m = 18432, k = 8192 17.3, 19.7; M = 1, m = 4096, k = 1024 3.5, 3.7;
+//   M = 16, m = 7168, k = 8192 10.6, 9.1; M = 64, m = 4096, k = 4096 10.1, 6.5; M = 40, m = 16384, k = 4096 13.5, 10.9.
+// Past m = 18432 the walk needs a second round of workgroups (M = 2, m = 22528, k = 8192 24.8, 20.1). Over 6512 shapes
+// (M = 1..64, m = 2048..24576), every weight from HBM, the rule takes 0.86 of the walk's time on average and at most 3%
+// more. Weights that stay in the Infinity Cache favour the tiles, whose reads it keeps (M = 64, m = 9216, k = 7168 16.8,
+// 11.6, from HBM 18.4, 16.8); right behind 768 MB of writes tiles are up to 25% slower than the walk (M = 8, m = 15360,
+// k = 4096).
 inline bool takes_walk(int64_t M, int64_t m, int64_t k) {
   if (M > 64 || k % 1024 || m > 18432) return false;
   const int64_t ktw = k / 1024;
   if (ktw != 1 && ktw != 2 && ktw != 4 && ktw != 7 && ktw != 8) return false;
-  const int64_t widest = M <= 16   ? (ktw == 1 ? 0 : 8192)  // the widest weights that the tiles take
-                         : M <= 32 ? (ktw == 1 ? 4096 : 8192)
-                         : ktw <= 4 ? 16384
-                         : M <= 48 ? 6144
-                                   : 8192;
+  const int64_t widest = ktw <= 2 && M <= 16 ? (ktw == 1 ? 0 : 8192)  // the widest weights that the tiles take
+                         : ktw <= 4          ? 16384
+                                             : 8192;
   return m > widest;
 }
 
@@ -61,7 +59,7 @@ inline int64_t small_tile_lds(const SmallTile& t, int64_t k) {
 // Infinity Cache) showed a bias. A tile's k group costs by its token subtiles (mt), its 16-row weight groups (n) and
 // their product, its output by the product; a tile past one per CU takes a further round. Tiles that fill the chip
 // are slower by a tenth, and by 40% more where K/512 is 7, 15 or 31: the weight rows of its waves then lie a power of
-// two less 4 KiB apart, and their requests meet on the same channels (32 x 128 to 80 x 128 tiles on 180 to 256 CUs:
+// two less 4 KiB apart, and their requests likely meet on the same channels (32 x 128 to 80 x 128 tiles on 180 to 256 CUs:
 // 1.3, 1.6 and 1.65 times the fit, against 1.1 to 1.2 at other K).
 inline double small_tile_us(const SmallTile& t, int64_t M, int64_t m, int64_t k) {
   const int64_t tiles = ceil_div(M, t.rows) * ceil_div(m, t.weights), kg = k / 512;
@@ -96,7 +94,7 @@ inline const SmallTile* best_small_tile(int64_t M, int64_t m, int64_t k, double*
 // A small tile is taken where the fit has it 10% shorter. Over the 6184 shapes the choice is within 0.5% of the fastest
 // kernel on average, and 3.3% slower than the ring at worst. Where the ring's last round is not full, its whole blocks
 // of the rounds before may stay on the ring and the rest go to small tiles, in a launch of their own behind the
-// ring's: taken where the fit has the two 13% shorter, which over 357 shapes with more than one round was 34 times,
+// ring's: taken where the fit has the two 13% shorter, which over 641 shapes with more than one round was 34 times,
 // 3% to 27% shorter measured and 13% on average (M = 1024, N = 9216, K = 7168, 288 tiles: 70.7 -> 59.3 us). With 5%
 // asked for it was 124 times, up to 14% slower (M = 531, N = 13312, K = 10240), and level at M = 2048, N = 9216,
 // K = 7168 (2.25 rounds).

@@ -277,10 +277,10 @@ def takes_walk(M: int, N: int, K: int) -> bool:
     """Whether the dense bf16 GEMM runs on the walk over the weights (csrc/pick.h: takes_walk, the same rule)."""
     if M > 64 or K % 1024 or K // 1024 not in WALK_KTW or N > 18432:
         return False
-    if M <= 32:
-        widest = (0 if M <= 16 else 4096) if K == 1024 else 8192
+    if K <= 2048 and M <= 16:
+        widest = 0 if K == 1024 else 8192
     else:
-        widest = 16384 if K <= 4096 else 6144 if M <= 48 else 8192
+        widest = 16384 if K <= 4096 else 8192
     return N > widest
 
 

@@ -90,14 +90,17 @@ def test_manifest_makes_the_same_dense_choice(pick):
                     assert L["shared_mem"] == tile_of(pick, M, N, K)[2] <= 163840
 
 
-# M, N, K, microseconds of the walk and of the tile that the fit picks (weights from HBM or from the Infinity Cache)
+# M, N, K, microseconds of the walk and of the tile that the fit picks, every weight from HBM
 WALK_TIMES = [
-    (16, 9216, 7168, 9.98, 11.11), (17, 9216, 8192, 12.59, 14.79), (32, 9216, 7168, 12.33, 14.21),
-    (16, 18432, 8192, 15.82, 19.64), (37, 17920, 7168, 17.99, 24.61), (64, 18432, 7168, 21.82, 27.17),
-    (40, 18432, 4096, 13.42, 14.36), (16, 9216, 1024, 4.09, 4.48), (1, 4096, 1024, 3.38, 3.61),
-    (64, 18432, 2048, 10.52, 11.53), (16, 7168, 8192, 10.12, 8.97), (64, 4096, 4096, 9.73, 6.09),
-    (64, 2048, 8192, 14.68, 6.35), (32, 1024, 4096, 6.71, 4.42), (48, 9216, 2048, 7.22, 5.26),
-    (64, 256, 1024, 5.61, 3.30), (2, 22528, 8192, 23.17, 21.79),
+    (16, 9216, 7168, 10.96, 11.33), (17, 9216, 8192, 13.51, 14.94), (32, 9216, 7168, 12.99, 14.38),
+    (16, 18432, 8192, 17.26, 19.67), (37, 17920, 7168, 18.85, 24.19), (64, 18432, 7168, 22.70, 26.65),
+    (40, 18432, 4096, 14.37, 13.70), (16, 9216, 1024, 4.12, 4.73), (1, 4096, 1024, 3.47, 3.74),
+    (64, 18432, 2048, 11.04, 11.64), (16, 7168, 8192, 10.58, 9.10), (64, 4096, 4096, 10.05, 6.53),
+    (64, 2048, 8192, 15.07, 7.36), (32, 1024, 4096, 7.09, 5.03), (48, 9216, 2048, 7.51, 5.91),
+    (64, 256, 1024, 5.83, 3.69), (2, 22528, 8192, 24.80, 20.10), (64, 9216, 7168, 18.35, 16.83),
+    (40, 16384, 4096, 13.50, 10.93), (40, 7168, 7168, 13.01, 13.22), (8, 14336, 2048, 5.74, 5.95),
+    (16, 12288, 4096, 8.74, 7.99), (32, 12288, 1024, 5.22, 4.98), (32, 9216, 4096, 9.24, 8.87),
+    (48, 8192, 8192, 15.54, 14.98),
 ]
 
 
