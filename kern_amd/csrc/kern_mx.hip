@@ -1879,8 +1879,9 @@ extern "C" __global__ __launch_bounds__(512) void kern_mx_gemm_bf16(const uint8_
 // so most of the chip idles until M * N holds some 200 of them. gemm_tiles covers the range below that: tiles of
 // 16*MT token rows x 16*NW*NF weight rows, one workgroup of NW waves each, wave w multiplying weight groups
 // [w*NF, +NF) of the tile with all of its token rows, k-tile after k-tile in one accumulator, so that every
-// result has the ring's bits. What bounds a tile is the operand bytes its CU can pull in (about 39 B a clock of the
-// 64 B the address path takes), so each operand byte is requested once per tile and many requests are in flight:
+// result has the ring's bits. What bounds a tile is the operand bytes its CU can pull in (50 KiB a k group of a 32 x 128
+// tile: M = 200, N = 4096, K = 7168 at 81 GB/s a CU, 62 with every weight from HBM, 2.8 us of the launch apart), so each
+// operand byte is requested once per tile and many requests are in flight:
 //   * weight fragments go straight into registers (a wave is the only one to use its fragments) and with them a
 //     scale dword per fragment and k group, S k groups (of 512) ahead. Default cache policy: with three weight
 //     copies in turn (M = 200, N = 4096, K = 7168) non-temporal loads took 14.2 us against 11.5 (the token
@@ -1893,10 +1894,11 @@ extern "C" __global__ __launch_bounds__(512) void kern_mx_gemm_bf16(const uint8_
 //     per k group (16 bytes of each row) they took as long as the activations: 17.8 against 14.9 us.
 // The k groups take the last steps of whole rounds of S, so that the last round needs no requests and none runs
 // past the end; the first steps of the first round (at most S - 1) send theirs to a zero-length resource.
-// Measured against the ring (one process, graph replays, three weight copies in turn, us): M = 40, N = 6144,
-// K = 3584 12.5 -> 6.4; M = 200, N = 4096, K = 7168 29.6 -> 12.3; M = 200, N = 7168, K = 2048 12.5 -> 7.9;
-// M = 128, N = 9216, K = 7168 30.4 -> 15.4; M = 1024, N = 4096, K = 7168 33.4 -> 28.6. A form that split K over
-// four waves and added the partial sums in LDS was within 10% either way and rounds differently.
+// Against the ring, us, graph replays over three weight copies in turn (from the Infinity Cache) and with every weight
+// from HBM: M = 40, N = 6144, K = 3584 12.5 -> 6.2 and 16.1 -> 8.0; M = 200, N = 4096, K = 7168 29.6 -> 11.6 and
+// 32.1 -> 14.3; M = 200, N = 7168, K = 2048 12.2 -> 8.8 and 12.9 -> 10.5; M = 128, N = 9216, K = 7168 29.8 -> 15.4 and
+// 38.5 -> 18.8; M = 1024, N = 4096, K = 7168 33.2 -> 29.0 and 39.5 -> 33.0. A form that split K over four waves and
+// added the partial sums in LDS was within 10% either way and rounds differently.
 template <int MT, int NW, int NF>
 struct TileCfg {
   static constexpr int S = NW * NF <= 4 && MT <= 2 ? 8 : (MT >= 5 || NF >= 2 ? 3 : 4);  // stages: k groups in flight
@@ -2356,10 +2358,11 @@ extern "C" __global__ __launch_bounds__(512) void kern_mx_gemm_mxfp8(const uint8
 //   * activations go through two k-tiles of the wave's LDS by buffer->LDS requests;
 //   * scales: the 16 bytes at (r % 32) * 16 of a 128-row block's 512 are the dwords of rows r % 32 + 32 i, so two
 //     requests bring a tile's weight scales (a dword request per 16 rows: 21.4 against 17.5 us).
-// The partial sums of the eight waves meet in LDS, in wave order. A CU then takes in about 37 B a clock, as in
-// gemm_tiles. Against kern_mx_gemm_mxfp8 (graph replays, three copies in turn, us): M = 72, N = 9216, K = 7168 55.4 ->
-// 17.3; M = 72, N = 2048, K = 7168 55 -> 10; M = 16, N = 4096, K = 2048 17.9 -> 3.2; M = 200, N = 4096, K = 7168
-// 57.8 -> 16.1; M = 500, N = 4096, K = 2048 22.0 -> 13.4.
+// The partial sums of the eight waves meet in LDS, in wave order. What bounds it is, as in gemm_tiles, the bytes a CU
+// pulls in (M = 72, N = 9216, K = 7168: 1.1 MB a workgroup at 71 GB/s, 48 with every weight from HBM). Against
+// kern_mx_gemm_mxfp8, us, three weight copies in turn and from HBM: M = 72, N = 9216, K = 7168 55.3 -> 18.0 and 65.4 ->
+// 25.6; M = 72, N = 2048, K = 7168 54.9 -> 9.6 and 63.9 -> 12.9; M = 16, N = 4096, K = 2048 17.8 -> 3.1 and 19.8 -> 4.6;
+// M = 200, N = 4096, K = 7168 58.1 -> 17.1 and 65.0 -> 19.8; M = 500, N = 4096, K = 2048 21.7 -> 13.1 and 24.1 -> 15.0.
 template <int MT, int NG>
 struct Tile8Cfg {
   static constexpr int NX = 2 * MT;                  // activation requests of a k-tile

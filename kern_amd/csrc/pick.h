@@ -95,7 +95,8 @@ inline const SmallTile* best_small_tile(int64_t M, int64_t m, int64_t k, double*
 // kernel on average, and 3.3% slower than the ring at worst. Where the ring's last round is not full, its whole blocks
 // of the rounds before may stay on the ring and the rest go to small tiles, in a launch of their own behind the
 // ring's: taken where the fit has the two 13% shorter, which over 641 shapes with more than one round was 34 times,
-// 3% to 27% shorter measured and 13% on average (M = 1024, N = 9216, K = 7168, 288 tiles: 70.7 -> 59.3 us). With 5%
+// 3% to 27% shorter measured and 13% on average (M = 1024, N = 9216, K = 7168, 288 tiles: 70.6 -> 57.2 us, weights from
+// HBM 83.0 -> 59.8). With 5%
 // asked for it was 124 times, up to 14% slower (M = 531, N = 13312, K = 10240), and level at M = 2048, N = 9216,
 // K = 7168 (2.25 rounds).
 struct DensePlan {
