@@ -70,13 +70,13 @@ inline double small_tile_us(const SmallTile& t, int64_t M, int64_t m, int64_t k)
   return us * (1 + 0.1 * full) * (kg >= 7 && (kg & (kg + 1)) == 0 ? 1 + 0.4 * full : 1);
 }
 // The ring's k group costs more as its tiles fill the chip (its clock falls). A last round that holds only tiles of a
-// partial block of rows costs their share of the rows, 0.3 at least (M = 531, N = 13312, K = 10240, 52 tiles of 19 rows
+// partial block of rows costs their share of the rows, 0.25 at least (M = 531, N = 13312, K = 10240, 52 tiles of 19 rows
 // after 208 whole ones: 65 us against the 94 of two whole rounds).
 inline double ring_us(int64_t M, int64_t m, int64_t k) {
   const int64_t nb = m / 256, tiles = ceil_div(M, 128) * nb, part = M % 128;
   double rounds = (double)ceil_div(tiles, 256);
   if (part && rounds > 1 && M / 128 * nb <= 256 * ((int64_t)rounds - 1))
-    rounds += std::max(0.3, (double)part / 128) - 1;
+    rounds += std::max(0.25, (double)part / 128) - 1;
   const double full = (double)tiles / 256, kg = (double)(k / 512);
   return 1.2 + rounds * (2.7 + 1.73 * kg) + full * (3.4 + 0.71 * kg);
 }
@@ -94,11 +94,10 @@ inline const SmallTile* best_small_tile(int64_t M, int64_t m, int64_t k, double*
 // A small tile is taken where the fit has it 10% shorter. Over the 6184 shapes the choice is within 0.5% of the fastest
 // kernel on average, and 3.3% slower than the ring at worst. Where the ring's last round is not full, its whole blocks
 // of the rounds before may stay on the ring and the rest go to small tiles, in a launch of their own behind the
-// ring's: taken where the fit has the two 13% shorter, which over 641 shapes with more than one round was 34 times,
-// 3% to 27% shorter measured and 13% on average (M = 1024, N = 9216, K = 7168, 288 tiles: 70.6 -> 57.2 us, weights from
-// HBM 83.0 -> 59.8). With 5%
-// asked for it was 124 times, up to 14% slower (M = 531, N = 13312, K = 10240), and level at M = 2048, N = 9216,
-// K = 7168 (2.25 rounds).
+// ring's: taken where the fit has the two 6% shorter, 13% at K < 4096 (below it the second launch weighs more than the
+// fit sees). Over 709 shapes with more than one round that was 97 times, 9% shorter on average and 0.8% longer at worst
+// (M = 1024, N = 9216, K = 7168, 288 tiles: 70.6 -> 57.2 us, weights from HBM 83.0 -> 59.8; M = 2048 there, 2.25 rounds
+// and close to the line: 126.1 -> 122.5 with its quantizer). With 5% asked for at every K some were 14% longer.
 struct DensePlan {
   int64_t ring_rows;
   const SmallTile* tile;  // for the rest of the rows, if any
@@ -111,7 +110,7 @@ inline DensePlan dense_plan(int64_t M, int64_t m, int64_t k) {
   const int64_t nb = m / 256, rounds = ceil_div(ceil_div(M, 128) * nb, 256);
   const int64_t blocks = 256 * (rounds - 1) / nb;  // whole blocks in all rounds but the last
   if (blocks > 0 && (tile = best_small_tile(M - 128 * blocks, m, k, &rest_us)) &&
-      ring_us(128 * blocks, m, k) + rest_us < 0.87 * ring)
+      ring_us(128 * blocks, m, k) + rest_us < (k >= 4096 ? 0.94 : 0.87) * ring)
     return {128 * blocks, tile};
   return {M, nullptr};
 }
