@@ -586,7 +586,7 @@ extern "C" int kern_mxfp4_gemv_bf16(const void* x, const void* w, const void* w_
     a.put(x), a.put(w), a.put(w_sf), a.put(y), a.put(M), a.put(N), a.put(K), a.put(gmax);
     return launch("kern_mx_gemv_bf16_rg", (uint32_t)(N / 16), 1, 1, 256, stream, a, 4u * (uint32_t)(gmax * M) * 1024u);
   }
-  if (kg <= 16) {
+  if (!kern::gemv_staged(M, N, K)) {
     // about 256 workgroups of 8 waves, each owning hb <= 9 half groups of 8 rows (at most five 16-row groups); a
     // wave owns a run of K/1024 k-tiles (rounded down or up where K is an odd multiple of 512: p{..}h) and holds
     // their x in registers, one k-tile at a time, passed through 4 KiB of LDS of its own
@@ -596,17 +596,11 @@ extern "C" int kern_mxfp4_gemv_bf16(const void* x, const void* w, const void* w_
     a.put(x), a.put(w), a.put(w_sf), a.put(y), a.put(M), a.put(N), a.put(K), a.put(hb);
     return launch(walk[kg - 1], (uint32_t)((H + hb - 1) / hb), 1, 1, 512, stream, a);
   }
-  // K > 8192 at M > 2: one workgroup per row group, x staged per workgroup in slices
-  // sb: k-tiles per wave whose slice of x is staged in LDS at once (at most four 16-byte pieces per lane,
+  // K > 8192 at M > 2, and some wider than the walk's one round: one workgroup per row group, x staged per workgroup in
+  // slices. sb: k-tiles per wave whose slice of x is staged in LDS at once (at most four 16-byte pieces per lane,
   // M * sb <= 16, sb divides K/512); nb: k-tiles per wave whose weights are in flight together (the
   // largest of the kernel's batch sizes dividing sb)
-  const int32_t kq = K / 512;
-  int32_t sb = 1;
-  for (int32_t cand = std::min(kq, 16 / M); cand >= 1; --cand)
-    if (kq % cand == 0) {
-      sb = cand;
-      break;
-    }
+  const int32_t sb = (int32_t)kern::gemv_slice(M, kg);
   int32_t nb = 1;
   for (int32_t cand : {7, 4, 2})
     if (sb % cand == 0) {
@@ -614,7 +608,7 @@ extern "C" int kern_mxfp4_gemv_bf16(const void* x, const void* w, const void* w_
       break;
     }
   // the x slice of every token, then the row group's scales (256 B per 512 of K)
-  const uint32_t lds = (uint32_t)M * (uint32_t)(sb * 1024 + 16) + (uint32_t)(kq * 256);
+  const uint32_t lds = (uint32_t)M * (uint32_t)(sb * 1024 + 16) + (uint32_t)(kg * 256);
   Args a;
   a.put(x), a.put(w), a.put(w_sf), a.put(y), a.put(M), a.put(N), a.put(K), a.put(nb), a.put(sb);
   return launch("kern_mx_gemv_bf16", (uint32_t)(N / 16), 1, 1, 256, stream, a, lds);

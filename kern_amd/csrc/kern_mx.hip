@@ -148,7 +148,7 @@ typedef __attribute__((address_space(1))) void glob_void_t;
 // non-gated) [N][K/2], in u8 w_sf (repacked), out bf16 y[M][N], i32 M, launch i32 N, i32 K, i32 nb, i32 sb.
 // Grid N/16, block 256, dynamic LDS M*(sb*1024 + 16) + K/2 bytes: one 16-row group per workgroup. Wave w
 // takes the 128-wide k-tiles kt = 4i + w (equal shares; its scale is byte w of each scale dword of the
-// group). Taken for K > 8192 at M > 2. x is consumed in slices of sb k-tiles per wave (sb divides K/512,
+// group). Taken for K > 8192 at M > 2 and some N > 18432 (gemv_staged). x is consumed in slices of sb k-tiles per wave (sb divides K/512,
 // M*sb <= 16), weights in rounds of nb fragments per wave (nb divides sb). Each slice of x, and with the
 // first slice the row group's
 // whole scale block, goes from memory straight into LDS (buffer loads to LDS, no registers); the round's

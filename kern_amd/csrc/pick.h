@@ -170,4 +170,26 @@ inline bool gemv_row_groups(int64_t M, int64_t N, int64_t K) {
   return N <= 4096 * std::min<int64_t>(2, 163840 / (x + gemv_row_group_lds(kg))) && (kg > 1 || N <= 4096);
 }
 
+// Past N = 18432 the walk's workgroups, nine half groups each, need a second round, and the slice-staging kernel
+// (kern_mx_gemv_bf16, one workgroup per row group at any N; K > 8192 runs on it anyway) may be ahead: M = 4, N = 19312,
+// K = 6144 14.7 against 18.7 us, but M = 16, N = 35904, K = 3584 26.1 against 18.2. Both times fitted to 13285 shapes
+// (M = 4..16, N up to 180000, every weight from HBM, the eleven K that took slice staging before the walk had them; rms
+// 5%). Over 8291 others of every K and M the choice takes 0.93 of the time of what they took then, at worst 11% more, and
+// more than 3% at 58 of them. At K = 512 * {2, 4, 8, 14, 16} the walk stays.
+inline int64_t gemv_slice(int64_t M, int64_t kg) {  // k-tiles per wave staged at once: divides kg, M * slice <= 16
+  int64_t sb = std::min<int64_t>(kg, 16 / M);
+  while (kg % sb) --sb;
+  return sb;
+}
+inline bool gemv_staged(int64_t M, int64_t N, int64_t K) {
+  const int64_t kg = K / 512, ktw = (kg + 1) / 2;
+  if (kg > 16) return true;
+  if (N <= 18432 || kg == 2 || kg == 4 || kg == 8 || kg == 14 || kg == 16) return false;
+  const double n = (double)N / 4096, m = (double)M, g = (double)kg, t = (double)ktw;
+  const double staged = 4.2 + n * (0.12 + 0.1256 * g + 0.0138 * g * m + 0.0096 * g / (double)gemv_slice(M, kg) - 0.006 * m);
+  const double walk =
+      2.8 + (double)ceil_div(N, 18432) * (0.5 + 0.69 * t + 0.0176 * t * m) + n * (-0.1 + 0.1 * g + 0.0009 * g * m);
+  return staged < 1.03 * walk;
+}
+
 }  // namespace kern

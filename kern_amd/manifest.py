@@ -217,6 +217,23 @@ def gemv_row_groups(M: int, N: int, K: int) -> bool:
     return M <= 3 or (N <= at_once and (kg > 1 or N <= 4096))
 
 
+def _gemv_slice(M: int, kg: int) -> int:
+    return next(c for c in range(min(kg, GEMV_MAX_ROWS // M), 0, -1) if kg % c == 0)
+
+
+def gemv_staged(M: int, N: int, K: int) -> bool:
+    """Whether a decode GEMV without row groups stages x in slices rather than walk (csrc/pick.h: gemv_staged)."""
+    kg = K // 512
+    if kg > GEMV_MAX_NKT:
+        return True
+    if N <= 18432 or kg in (2, 4, 8, 14, 16):
+        return False
+    n, t = N / 4096, _ceil(kg, 2)
+    staged = 4.2 + n * (0.12 + 0.1256 * kg + 0.0138 * kg * M + 0.0096 * kg / _gemv_slice(M, kg) - 0.006 * M)
+    walk = 2.8 + _ceil(N, 18432) * (0.5 + 0.69 * t + 0.0176 * t * M) + n * (-0.1 + 0.1 * kg + 0.0009 * kg * M)
+    return staged < 1.03 * walk
+
+
 def _gemv_launch(N: int, K: int, M: int, rows_var: str) -> dict:
     """The launch kern_mxfp4_gemv_bf16 makes for M rows of x [M][K] against weights [N][K/2] (capi.cpp)."""
     kg = K // 512
@@ -232,13 +249,13 @@ def _gemv_launch(N: int, K: int, M: int, rows_var: str) -> dict:
         return {"entry": "kern_mx_gemv_bf16_rg", "params": params + ["i32"], "block": [256, 1, 1],
                 "grid": row_groups, "shared_mem": {"mul": [rows_var, 4 * gmax * 1024]},
                 "args": args + [{"i32": gmax}]}
-    if kg <= GEMV_MAX_NKT:
+    if not gemv_staged(M, N, K):
         H = N // 8
         hb = min(9, _ceil(H, 256))
         return {"entry": f"kern_mx_gemv_bf16_p{_ceil(kg, 2)}{'h' if kg % 2 else ''}", "params": params + ["i32"],
                 "block": [512, 1, 1], "grid": [_ceil(H, hb), 1, 1], "args": args + [{"i32": hb}]}
-    # K > 8192: x staged in slices of sb k-tiles per wave, nb k-tiles of weights in flight together
-    sb = next(c for c in range(min(kg, GEMV_MAX_ROWS // M), 0, -1) if kg % c == 0)
+    # x staged in slices of sb k-tiles per wave, nb k-tiles of weights in flight together
+    sb = _gemv_slice(M, kg)
     nb = next((c for c in (7, 4, 2) if sb % c == 0), 1)
     return {"entry": "kern_mx_gemv_bf16", "params": params + ["i32", "i32"], "block": [256, 1, 1],
             "grid": row_groups, "shared_mem": M * (sb * 1024 + 16) + kg * 256, "args": args + [{"i32": nb}, {"i32": sb}]}

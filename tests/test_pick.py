@@ -34,6 +34,7 @@ extern "C" const char* entry(int i, int kind) {
   return kind ? kSmallTiles[i].e4m3 : kSmallTiles[i].bf16;
 }
 extern "C" int gemv(int64_t M, int64_t N, int64_t K) { return gemv_row_groups(M, N, K); }
+extern "C" int staged(int64_t M, int64_t N, int64_t K) { return gemv_staged(M, N, K); }
 extern "C" int64_t gemv_lds(int64_t kg, int64_t, int64_t) { return gemv_row_group_lds(kg); }
 extern "C" int64_t ring(int64_t M, int64_t m, int64_t k) { return dense_plan(M, m, k).ring_rows; }
 """
@@ -48,7 +49,7 @@ def pick(tmp_path_factory):
                     str(d / "shim.so")], check=True)
     L = ctypes.CDLL(str(d / "shim.so"))
     L.ring.restype = L.gemv_lds.restype = ctypes.c_int64
-    for f in (L.takes, L.ring, L.tile8, L.gemv, L.gemv_lds):
+    for f in (L.takes, L.ring, L.tile8, L.gemv, L.staged, L.gemv_lds):
         f.argtypes = [ctypes.c_int64] * 3
     L.tile.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_void_p] * 3
     return L
@@ -196,6 +197,9 @@ def test_manifest_makes_the_same_gemv_choice(pick):
         for kg in range(1, 18):
             for N in (16, 4080, 4096, 4112, 8192, 8208, 18432):
                 assert bool(pick.gemv(M, N, 512 * kg)) == mf.gemv_row_groups(M, N, 512 * kg), (M, N, kg)
+                assert bool(pick.staged(M, N, 512 * kg)) == mf.gemv_staged(M, N, 512 * kg), (M, N, kg)
+            for N in range(18432, 80000, 1616):
+                assert bool(pick.staged(M, N, 512 * kg)) == mf.gemv_staged(M, N, 512 * kg), (M, N, kg)
 
 
 @pytest.mark.parametrize("M,N,K,row_groups", [(5, 8192, 7680, False), (5, 4096, 7680, True), (1, 18432, 7168, True),
@@ -203,6 +207,15 @@ def test_manifest_makes_the_same_gemv_choice(pick):
                                               (16, 7168, 512, False)])
 def test_gemv_routes(pick, M, N, K, row_groups):
     assert bool(pick.gemv(M, N, K)) == row_groups
+
+
+@pytest.mark.parametrize("M,N,K,staged,walk", [
+    (4, 19312, 6144, 14.66, 18.74), (4, 19616, 5632, 15.31, 18.27), (5, 18864, 4608, 13.41, 15.88),
+    (6, 19856, 6656, 17.74, 20.94), (6, 18592, 7680, 19.78, 23.17), (7, 20240, 2560, 9.55, 11.10),
+    (7, 18896, 4608, 13.86, 16.00)])
+def test_gemv_stages_slices_where_the_walk_is_slower(pick, M, N, K, staged, walk):
+    """Slice staging is what every such call ran on before the walk had these lengths (microseconds of both)."""
+    assert walk > 1.03 * staged and not pick.gemv(M, N, K) and pick.staged(M, N, K)
 
 
 @pytest.mark.parametrize("K", [1024, 2048, 4096, 7168, 8192])
