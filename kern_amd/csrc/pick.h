@@ -21,15 +21,17 @@ inline int64_t walk_half_groups(int64_t m) { return std::min<int64_t>(9, ceil_di
 // workgroups each read all of the activations, so more rows and narrow weights favour the tiles. Walk, tile in us:
 //   M = 32, m = 9216, k = 7168 13.0, 14.4; M = 16, m = 18432, k = 8192 17.3, 19.7; M = 1, m = 4096, k = 1024 3.5, 3.7;
 //   M = 16, m = 7168, k = 8192 10.6, 9.1; M = 64, m = 4096, k = 4096 10.1, 6.5; M = 40, m = 16384, k = 4096 13.5, 10.9.
-// Past m = 18432 the walk needs a second round of workgroups (M = 2, m = 22528, k = 8192 24.8, 20.1). Over 6512 shapes
+// Past m = 18432 the walk needs a second round of workgroups (M = 2, m = 22528, k = 8192 24.8, 20.1) and is ahead only
+// where its rounds are nearly full (0.86), at M <= 16 and k >= 7168 (M = 4, m = 33280, k = 7168 24.4, 32.9). Over 6512 shapes
 // (M = 1..64, m = 2048..24576), every weight from HBM, the rule takes 0.86 of the walk's time on average and at most 3%
 // more. Weights that stay in the Infinity Cache favour the tiles, whose reads it keeps (M = 64, m = 9216, k = 7168 16.8,
 // 11.6, from HBM 18.4, 16.8); right behind 768 MB of writes tiles are up to 25% slower than the walk (M = 8, m = 15360,
 // k = 4096).
 inline bool takes_walk(int64_t M, int64_t m, int64_t k) {
-  if (M > 64 || k % 1024 || m > 18432) return false;
+  if (M > 64 || k % 1024) return false;
   const int64_t ktw = k / 1024;
   if (ktw != 1 && ktw != 2 && ktw != 4 && ktw != 7 && ktw != 8) return false;
+  if (m > 18432) return M <= 16 && ktw >= 7 && m >= 15852 * ceil_div(m, 18432);
   const int64_t widest = ktw <= 2 && M <= 16 ? (ktw == 1 ? 0 : 8192)  // the widest weights that the tiles take
                          : ktw <= 4          ? 16384
                                              : 8192;
@@ -91,8 +93,10 @@ inline const SmallTile* best_small_tile(int64_t M, int64_t m, int64_t k, double*
   return best;
 }
 // The rows the ring takes, a whole number of its 128-row blocks or all of them (the small tiles take the rest).
-// A small tile is taken where the fit has it 10% shorter. Over the 6184 shapes the choice is within 0.5% of the fastest
-// kernel on average, and 3.3% slower than the ring at worst. Where the ring's last round is not full, its whole blocks
+// A small tile is taken where the fit has it 10% shorter, at K > 8192 and one round of the ring its weights counted at
+// 4 TB/s at most (the ring's come from HBM at up to 5: M = 2, m = 33280, k = 12288 46.1 against 52.6 us). Over the 6184 shapes the choice is within 0.5% of the
+// fastest kernel on average, and 3.3% slower than the ring at worst; over 8462 with m up to
+// 160000 or k up to 65536 it is more than 3% slower than the ring or the walk at 2% of them, 15% at worst. Where the ring's last round is not full, its whole blocks
 // of the rounds before may stay on the ring and the rest go to small tiles, in a launch of their own behind the
 // ring's: taken where the fit has the two 6% shorter, 13% at K < 4096 (below it the second launch weighs more than the
 // fit sees). Over 709 shapes with more than one round that was 97 times, 9% shorter on average and 0.8% longer at worst
@@ -106,8 +110,9 @@ inline DensePlan dense_plan(int64_t M, int64_t m, int64_t k) {
   double us = 0, rest_us = 0;
   const double ring = ring_us(M, m, k);
   const SmallTile* tile = best_small_tile(M, m, k, &us);
-  if (tile && us < 0.9 * ring) return {0, tile};
   const int64_t nb = m / 256, rounds = ceil_div(ceil_div(M, 128) * nb, 256);
+  if (rounds == 1 && k > 8192) us = std::max(us, (double)(m * k) * (17.0 / 32) / 4e6);
+  if (tile && us < 0.9 * ring) return {0, tile};
   const int64_t blocks = 256 * (rounds - 1) / nb;  // whole blocks in all rounds but the last
   if (blocks > 0 && (tile = best_small_tile(M - 128 * blocks, m, k, &rest_us)) &&
       ring_us(128 * blocks, m, k) + rest_us < (k >= 4096 ? 0.94 : 0.87) * ring)

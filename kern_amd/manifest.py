@@ -292,8 +292,10 @@ SMALL_TILES = ((16, 32, 2, 8), (16, 64, 4, 8), (16, 128, 8, 4), (32, 128, 8, 4),
 
 def takes_walk(M: int, N: int, K: int) -> bool:
     """Whether the dense bf16 GEMM runs on the walk over the weights (csrc/pick.h: takes_walk, the same rule)."""
-    if M > 64 or K % 1024 or K // 1024 not in WALK_KTW or N > 18432:
+    if M > 64 or K % 1024 or K // 1024 not in WALK_KTW:
         return False
+    if N > 18432:
+        return M <= 16 and K >= 7168 and N >= 15852 * _ceil(N, 18432)
     if K <= 2048 and M <= 16:
         widest = 0 if K == 1024 else 8192
     else:

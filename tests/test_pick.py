@@ -81,7 +81,7 @@ def test_every_tile_has_an_entry(pick):
 
 def test_manifest_makes_the_same_dense_choice(pick):
     for K in (1024, 2048, 4096, 7168, 8192):
-        for N in [256 * i for i in range(1, 40)] + [14336, 16384, 16640, 18432, 18688, 24576]:
+        for N in [256 * i for i in range(1, 40)] + [14336, 16384, 16640, 18432, 18688, 24576, 33024, 33280, 36864]:
             for M in (1, 2, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64):
                 want = f"kern_mx_gemm_bf16_s{K // 1024}" if pick.takes(M, N, K) else \
                     "kern_mx_gemm_bf16_t%dx%d" % tile_of(pick, M, N, K)[:2]
@@ -93,6 +93,7 @@ def test_manifest_makes_the_same_dense_choice(pick):
 
 # M, N, K, microseconds of the walk and of the tile that the fit picks, every weight from HBM
 WALK_TIMES = [
+    (4, 33280, 7168, 24.42, 32.87), (8, 35072, 7168, 25.28, 33.58), (1, 33536, 7168, 24.48, 32.58),
     (16, 9216, 7168, 10.96, 11.33), (17, 9216, 8192, 13.51, 14.94), (32, 9216, 7168, 12.99, 14.38),
     (16, 18432, 8192, 17.26, 19.67), (37, 17920, 7168, 18.85, 24.19), (64, 18432, 7168, 22.70, 26.65),
     (40, 18432, 4096, 14.37, 13.70), (16, 9216, 1024, 4.12, 4.73), (1, 4096, 1024, 3.47, 3.74),
@@ -119,6 +120,7 @@ RING_TIMES = [
     (567, 5632, 7680, 34.74, 40.84), (3360, 768, 7680, 32.02, 36.81), (2394, 1024, 7680, 31.98, 36.64),
     (3235, 2560, 1536, 19.59, 21.91), (1025, 7680, 7680, 57.18, 79.54), (555, 6400, 15872, 63.8, 78.72),
     (550, 13568, 3584, 32.91, 41.54), (779, 9728, 4608, 37.74, 45.26), (305, 11776, 7680, 38.26, 45.48),
+    (2, 33280, 12288, 46.14, 52.59), (6, 34048, 12800, 50.39, 57.45), (8, 35072, 8704, 36.87, 41.76),
     (1191, 7680, 512, 13.28, 15.46), (3885, 3072, 3072, 34.84, 37.59), (1813, 13312, 4608, 83.44, 96.02),
 ]
 
