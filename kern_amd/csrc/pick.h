@@ -93,15 +93,16 @@ inline const SmallTile* best_small_tile(int64_t M, int64_t m, int64_t k, double*
   return best;
 }
 // The rows the ring takes, a whole number of its 128-row blocks or all of them (the small tiles take the rest).
-// A small tile is taken where the fit has it 10% shorter, at K > 8192 and one round of the ring its weights counted at
-// 4 TB/s at most (the ring's come from HBM at up to 5: M = 2, m = 33280, k = 12288 46.1 against 52.6 us). Over the 6184 shapes the choice is within 0.5% of the
-// fastest kernel on average, and 3.3% slower than the ring at worst; over 8462 with m up to
-// 160000 or k up to 65536 it is more than 3% slower than the ring or the walk at 2% of them, 15% at worst. Where the ring's last round is not full, its whole blocks
-// of the rounds before may stay on the ring and the rest go to small tiles, in a launch of their own behind the
-// ring's: taken where the fit has the two 6% shorter, 13% at K < 4096 (below it the second launch weighs more than the
-// fit sees). Over 709 shapes with more than one round that was 97 times, 9% shorter on average and 0.8% longer at worst
-// (M = 1024, N = 9216, K = 7168, 288 tiles: 70.6 -> 57.2 us, weights from HBM 83.0 -> 59.8; M = 2048 there, 2.25 rounds
-// and close to the line: 126.1 -> 122.5 with its quantizer). With 5% asked for at every K some were 14% longer.
+// A small tile is taken where the fit has it 10% shorter; at K > 8192 and one round of the ring its weights count at
+// 4 TB/s at most (the ring's come from HBM at up to 5: M = 2, m = 33280, k = 12288 46.1 against 52.6 us). Over the 6184
+// shapes the choice is within 0.5% of the fastest kernel on average, and 3.3% slower than the ring at worst; over 8462
+// with m up to 160000 or k up to 65536 it is more than 3% slower than the ring or the walk at 2%, 15% at worst.
+// Where the ring's last round is not full, its whole blocks of the rounds before may stay on the ring and the rest go to
+// small tiles, in a launch of their own behind the ring's: taken where the fit has the two 6% shorter, 13% at K < 4096
+// (there the second launch weighs more than the fit sees). Over 709 shapes with more than one round that was 97 times, 9%
+// shorter on average and 0.8% longer at worst (M = 1024, N = 9216, K = 7168, 288 tiles: 70.6 -> 57.2 us, weights from HBM
+// 83.0 -> 59.8; M = 2048 there, 2.25 rounds and close to the line: 126.1 -> 122.5 with its quantizer). With 5% asked for
+// at every K some were 14% longer.
 struct DensePlan {
   int64_t ring_rows;
   const SmallTile* tile;  // for the rest of the rows, if any
@@ -126,7 +127,8 @@ inline DensePlan dense_plan(int64_t M, int64_t m, int64_t k) {
 // the fit has it 15% shorter (its error), in three and more rounds 28% (there its error grows: M = 524, N = 7296,
 // K = 960, 1254 tiles of 48 x 64 took 23.0 us against the large tiles' 18.6). Over 8582 shapes (M = 1..6144,
 // N = 16..20480, K = 128..16384) the choice takes 0.34 of the large tiles' time, is within 1% of the fastest on average,
-// and never slower than the large tiles; with 15% at any number of rounds 16 were, by up to 24%.
+// and never slower than the large tiles; with 15% at any number of rounds 16 were, by up to 24%. Over 3353 with N up to
+// 160000 or K up to 65536 25 are more than 3% slower, 17% at worst.
 struct SmallTile8 {
   int rows, weights;
   const char* entry;
