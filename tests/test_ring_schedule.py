@@ -23,6 +23,7 @@ staged x by buffer->LDS requests one k-tile ahead with a fixed count (the form d
 mismatch): the last k-tile of every wave has fewer weight requests behind its x request than the fixed
 count assumes.
 """
+import functools
 import itertools
 
 import pytest
@@ -416,9 +417,9 @@ def test_gemv_staged_x_variant_fixed_count_is_short(KTW):
 # ------------------------------------------------------------------------------------------ the code object
 
 
-def _disassembly(fn):
+@functools.lru_cache(maxsize=1)
+def _code_object_text():
     import os
-    import re
     import subprocess
 
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -426,8 +427,13 @@ def _disassembly(fn):
     objdump = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "llvm-objdump")
     if not (os.path.exists(hsaco) and os.path.exists(objdump)):
         pytest.skip("needs the built code object and llvm-objdump")
-    text = subprocess.run([objdump, "-d", "--mcpu=gfx950", hsaco], capture_output=True, text=True,
-                          check=True).stdout
+    return subprocess.run([objdump, "-d", "--mcpu=gfx950", hsaco], capture_output=True, text=True, check=True).stdout
+
+
+def _disassembly(fn):
+    import re
+
+    text = _code_object_text()
     out, on = [], False
     for line in text.splitlines():
         if line.endswith(f"<{fn}>:"):
